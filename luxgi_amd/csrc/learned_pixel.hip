@@ -26,8 +26,8 @@
 // the activations passed between layers through LDS. Training: the backward of a scaled pass in
 // gather form (a centre kernel keeps each filtered pixel's dL/d(out) / sum of weights and its
 // luminance factor; a gather kernel adds each pixel's share of its neighbours' taps, no atomics)
-// and the MLP's backward per pixel with the parameter gradient summed per block in LDS and the
-// blocks' partial sums added in block order (deterministic). The weights' dependence on the input
+// and the MLP's backward on the matrix units with the parameter gradient summed per wave, block
+// and grid in a fixed order (deterministic). The weights' dependence on the input
 // colour (luminance, the variance behind phi) is held fixed in the backward.
 #include "svgf_common.hpp"
 
@@ -309,126 +309,232 @@ __global__ __launch_bounds__(256) void lp_pass_gather_kernel(LpPassArgs A, const
 }
 
 // ---------------------------------------------------------------------------------------------
-// Backward of the MLP. A block takes chunks of 64 pixels: lanes 0..63 run one pixel each (the
-// forward with FP16-rounded operands, then dL/do = dL/ds * s inside the clamp, dL/dh2, dL/dh1)
-// into LDS, then every lane sums its parameters' terms over the chunk. Each block writes its sums
-// to partial[block]; lp_reduce_kernel adds the blocks' partials in order into the gradient.
+// Backward of the MLP, on the matrix units, 16 pixels per wave and step. With the lane layouts
+// above, D of a layer leaves lane (g, col) with units 4g + v and 16 + 4g + v of pixel col; the next
+// contraction over units takes them as they are, with its K slots numbered to match (FP16
+// 16x16x32: slot 8g + j is unit 4g + j, or 16 + 4g + j - 4; FP32 16x16x4: step (mt, v) has unit
+// 16 mt + 4g + v in slot g), so the activations and the gradients pass from layer to layer in
+// registers and only the weight fragments carry the permutation. The forward is recomputed as
+// lp_forward_kernel does it (FP16 operands, FP32 sums); everything that holds a gradient is FP32
+// (v_mfma_f32_16x16x4f32). The parameter gradients contract over pixels: the wave turns its 16
+// pixels' gradients and activations around through its own LDS rows and keeps the 1,637 sums
+// in accumulators over all its pixels. A block adds its waves in wave order into
+// partial[block]; lp_reduce_kernel adds the blocks, in an order that is fixed too.
+//
+// Bound: the FP32 matrix rate (56 MFMAs of 32 cycles per 16 pixels: 24 us for 960x540) and the
+// LDS turn. One lane per pixel with the per-parameter sums read from LDS (64 of a block's 256
+// lanes busy in the layers, a scalar chain per parameter) took 2,553 us at 960x540, and the
+// training step there 3.14 ms against 0.60 ms with this form.
 // ---------------------------------------------------------------------------------------------
-constexpr int kLpChunk = 64;
 constexpr int kLpBwdBlocks = 240;
+constexpr int kLpBwdWaves = 8;     // two waves per SIMD of the block's CU
+constexpr int kLpRow = 17;         // LDS row of 16 pixels, padded by one bank
 
-struct LpBackwardLds {
-    float f[kLpChunk][kLpIn];
-    float h1[kLpChunk][kLpHid + 1];
-    float h2[kLpChunk][kLpHid + 1];
-    float g1[kLpChunk][kLpHid + 1];
-    float g2[kLpChunk][kLpHid + 1];
-    float go[kLpChunk][kLpOut];
+// one wave's 16 pixels, [unit][pixel]
+struct LpTurn {
+    float f[16][kLpRow];            // 12 features, then 1 (the bias column of layer 1), then 0
+    float h1[kLpHid][kLpRow], h2[kLpHid][kLpRow], g1[kLpHid][kLpRow], g2[kLpHid][kLpRow];
+    float go[16][kLpRow];           // 5 outputs, then 0
+};
+union LpBackwardLds {
+    LpTurn turn[kLpBwdWaves];
+    float sums[kLpBwdWaves][kLpParams];
 };
 
-__device__ __forceinline__ float lp_q(float v) { return (float)(_Float16)v; }
+typedef float lp_float4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-__global__ __launch_bounds__(256) void lp_mlp_backward_kernel(const float* __restrict__ P, long long N,
-                                                              const float* __restrict__ feat,
-                                                              const float* __restrict__ gScales,
-                                                              const float* __restrict__ scales,
-                                                              float* __restrict__ partial) {
+__device__ __forceinline__ float lp_q(float v) { return (float)(_Float16)v; }
+__device__ __forceinline__ lp_float4 lp_mfma4(float a, float b, lp_float4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(64 * kLpBwdWaves) void lp_mlp_backward_kernel(const float* __restrict__ P, long long N,
+                                                                           const float* __restrict__ feat,
+                                                                           const float* __restrict__ gScales,
+                                                                           const float* __restrict__ scales,
+                                                                           float* __restrict__ partial) {
     __shared__ LpBackwardLds lds;
-    const int tid = threadIdx.x;
-    constexpr int kPer = (kLpParams + 255) / 256;
-    float acc[kPer];
-    for (int i = 0; i < kPer; ++i) acc[i] = 0.0f;
-    const long long chunks = (N + kLpChunk - 1) / kLpChunk;
-    for (long long c = blockIdx.x; c < chunks; c += gridDim.x) {
-        if (tid < kLpChunk) {
-            const long long p = c * kLpChunk + tid;
-            float f[kLpIn], h1[kLpHid], h2[kLpHid], go[kLpOut];
-            bool m1[kLpHid], m2[kLpHid];
-            if (p < N) {
-                for (int i = 0; i < kLpIn; ++i) f[i] = lp_q(feat[p * kLpIn + i]);
-                for (int j = 0; j < kLpHid; ++j) {
-                    float a = P[kLpB1 + j];
-                    for (int i = 0; i < kLpIn; ++i) a += lp_q(P[kLpW1 + j * kLpIn + i]) * f[i];
-                    m1[j] = a > 0.0f;
-                    h1[j] = lp_q(fmaxf(a, 0.0f));
-                }
-                for (int j = 0; j < kLpHid; ++j) {
-                    float a = P[kLpB2 + j];
-                    for (int i = 0; i < kLpHid; ++i) a += lp_q(P[kLpW2 + j * kLpHid + i]) * h1[i];
-                    m2[j] = a > 0.0f;
-                    h2[j] = lp_q(fmaxf(a, 0.0f));
-                }
-                for (int j = 0; j < kLpOut; ++j) {
-                    float a = P[kLpB3 + j];
-                    for (int i = 0; i < kLpHid; ++i) a += lp_q(P[kLpW3 + j * kLpHid + i]) * h2[i];
-                    const size_t e = (size_t)j * N + p;
-                    go[j] = (a > -kLpClamp && a < kLpClamp) ? gScales[e] * scales[e] : 0.0f;
-                }
-            } else {
-                for (int i = 0; i < kLpIn; ++i) f[i] = 0.0f;
-                for (int j = 0; j < kLpHid; ++j) {
-                    h1[j] = h2[j] = 0.0f;
-                    m1[j] = m2[j] = false;
-                }
-                for (int j = 0; j < kLpOut; ++j) go[j] = 0.0f;
-            }
-            float gh2[kLpHid], gh1[kLpHid];
-            for (int i = 0; i < kLpHid; ++i) {
-                float s = 0.0f;
-                for (int j = 0; j < kLpOut; ++j) s += go[j] * lp_q(P[kLpW3 + j * kLpHid + i]);
-                gh2[i] = m2[i] ? s : 0.0f;
-            }
-            for (int i = 0; i < kLpHid; ++i) {
-                float s = 0.0f;
-                for (int j = 0; j < kLpHid; ++j) s += gh2[j] * lp_q(P[kLpW2 + j * kLpHid + i]);
-                gh1[i] = m1[i] ? s : 0.0f;
-            }
-            for (int i = 0; i < kLpIn; ++i) lds.f[tid][i] = f[i];
-            for (int i = 0; i < kLpHid; ++i) {
-                lds.h1[tid][i] = h1[i];
-                lds.h2[tid][i] = h2[i];
-                lds.g1[tid][i] = gh1[i];
-                lds.g2[tid][i] = gh2[i];
-            }
-            for (int j = 0; j < kLpOut; ++j) lds.go[tid][j] = go[j];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int col = lane & 15, g = lane >> 4;
+    // forward weight fragments (FP16), biases of the units this lane's D holds
+    lp_half4 a1[2];
+    lp_half8 a2[2], a3;
+    lp_float4 b1v[2], b2v[2], b3v;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+        const int u = mt * 16 + col;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = 4 * g + j;
+            a1[mt][j] = (_Float16)(k < kLpIn ? P[kLpW1 + u * kLpIn + k] : 0.0f);
+            a2[mt][j] = (_Float16)P[kLpW2 + u * kLpHid + k];
+            a2[mt][4 + j] = (_Float16)P[kLpW2 + u * kLpHid + 16 + k];
+            b1v[mt][j] = P[kLpB1 + mt * 16 + k];
+            b2v[mt][j] = P[kLpB2 + mt * 16 + k];
         }
-        __syncthreads();
-        for (int i = 0; i < kPer; ++i) {
-            const int k = tid + i * 256;
-            if (k >= kLpParams) break;
-            float s = 0.0f;
-            if (k < kLpB1) {
-                const int j = (k - kLpW1) / kLpIn, ii = (k - kLpW1) % kLpIn;
-                for (int p = 0; p < kLpChunk; ++p) s += lds.g1[p][j] * lds.f[p][ii];
-            } else if (k < kLpW2) {
-                for (int p = 0; p < kLpChunk; ++p) s += lds.g1[p][k - kLpB1];
-            } else if (k < kLpB2) {
-                const int j = (k - kLpW2) / kLpHid, ii = (k - kLpW2) % kLpHid;
-                for (int p = 0; p < kLpChunk; ++p) s += lds.g2[p][j] * lds.h1[p][ii];
-            } else if (k < kLpW3) {
-                for (int p = 0; p < kLpChunk; ++p) s += lds.g2[p][k - kLpB2];
-            } else if (k < kLpB3) {
-                const int j = (k - kLpW3) / kLpHid, ii = (k - kLpW3) % kLpHid;
-                for (int p = 0; p < kLpChunk; ++p) s += lds.go[p][j] * lds.h2[p][ii];
-            } else {
-                for (int p = 0; p < kLpChunk; ++p) s += lds.go[p][k - kLpB3];
-            }
-            acc[i] += s;
-        }
-        __syncthreads();
     }
-    for (int i = 0; i < kPer; ++i) {
-        const int k = tid + i * 256;
-        if (k < kLpParams) partial[(size_t)blockIdx.x * kLpParams + k] = acc[i];
+    // the transposed weights of the gradient's way back, [unit of the layer below][unit], step (mt, v)
+    float t3[2][4], t2[2][2][4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int k = 4 * g + v;
+        a3[v] = (_Float16)(col < kLpOut ? P[kLpW3 + col * kLpHid + k] : 0.0f);
+        a3[4 + v] = (_Float16)(col < kLpOut ? P[kLpW3 + col * kLpHid + 16 + k] : 0.0f);
+        b3v[v] = k < kLpOut ? P[kLpB3 + k] : 0.0f;
+#pragma unroll
+        for (int mo = 0; mo < 2; ++mo) {
+            t3[mo][v] = k < kLpOut ? lp_q(P[kLpW3 + k * kLpHid + mo * 16 + col]) : 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) t2[mo][mt][v] = lp_q(P[kLpW2 + (mt * 16 + k) * kLpHid + mo * 16 + col]);
+        }
+    }
+    const lp_float4 zero = {0.f, 0.f, 0.f, 0.f};
+    lp_float4 w1[2] = {zero, zero}, w2[2][2] = {{zero, zero}, {zero, zero}}, w3[2] = {zero, zero};
+    lp_float4 sb2[2] = {zero, zero}, sb3 = zero;
+    LpTurn& T = lds.turn[wave];
+    const long long tiles = (N + 15) / 16;
+    for (long long tile = (long long)blockIdx.x * kLpBwdWaves + wave; tile < tiles;
+         tile += (long long)gridDim.x * kLpBwdWaves) {
+        const long long p = tile * 16 + col;
+        const bool in = p < N;
+        lp_float4 f = zero;
+        if (in && g < 3) f = *reinterpret_cast<const lp_float4_a4*>(feat + p * kLpIn + 4 * g);
+        float gs[4], sc[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const bool on = in && 4 * g + v < kLpOut;
+            const size_t e = (size_t)(4 * g + v) * N + p;
+            gs[v] = on ? gScales[e] : 0.0f;
+            sc[v] = on ? scales[e] : 0.0f;
+        }
+        lp_half4 bf;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bf[j] = (_Float16)f[j];
+        lp_half8 q1, q2;
+        lp_float4 d1[2], d2[2];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+            d1[mt] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1[mt], bf, b1v[mt], 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) q1[mt * 4 + v] = (_Float16)fmaxf(d1[mt][v], 0.0f);
+        }
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+            d2[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a2[mt], q1, b2v[mt], 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) q2[mt * 4 + v] = (_Float16)fmaxf(d2[mt][v], 0.0f);
+        }
+        const lp_float4 o = __builtin_amdgcn_mfma_f32_16x16x32_f16(a3, q2, b3v, 0, 0, 0);
+        lp_float4 go;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) go[v] = (o[v] > -kLpClamp && o[v] < kLpClamp) ? gs[v] * sc[v] : 0.0f;
+        lp_float4 g2[2] = {zero, zero}, g1[2] = {zero, zero};
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int mo = 0; mo < 2; ++mo) g2[mo] = lp_mfma4(t3[mo][v], go[v], g2[mo]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) g2[mt][v] = d2[mt][v] > 0.0f ? g2[mt][v] : 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int mo = 0; mo < 2; ++mo) g1[mo] = lp_mfma4(t2[mo][mt][v], g2[mt][v], g1[mo]);
+        // turn: [unit][pixel], written by pixel and read by unit (the wave's own rows: no barrier, the
+        // LDS serves a wave's accesses in order)
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int u = mt * 16 + 4 * g + v;
+                g1[mt][v] = d1[mt][v] > 0.0f ? g1[mt][v] : 0.0f;
+                T.g1[u][col] = g1[mt][v];
+                T.g2[u][col] = g2[mt][v];
+                T.h1[u][col] = (float)q1[mt * 4 + v];
+                T.h2[u][col] = (float)q2[mt * 4 + v];
+            }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            T.f[4 * g + v][col] = g < 3 ? (float)bf[v] : (v == 0 ? 1.0f : 0.0f);
+            T.go[4 * g + v][col] = go[v];
+        }
+        sb2[0] += g2[0];
+        sb2[1] += g2[1];
+        sb3 += go;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {  // pixels 4s + g
+            const int px = 4 * s + g;
+            const float bF = T.f[col][px], aO = T.go[col][px];
+            const float h1a = T.h1[col][px], h1b = T.h1[16 + col][px], h2a = T.h2[col][px], h2b = T.h2[16 + col][px];
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+                const float x1 = T.g1[mt * 16 + col][px], x2 = T.g2[mt * 16 + col][px];
+                w1[mt] = lp_mfma4(x1, bF, w1[mt]);
+                w2[mt][0] = lp_mfma4(x2, h1a, w2[mt][0]);
+                w2[mt][1] = lp_mfma4(x2, h1b, w2[mt][1]);
+            }
+            w3[0] = lp_mfma4(aO, h2a, w3[0]);
+            w3[1] = lp_mfma4(aO, h2b, w3[1]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    }
+    __syncthreads();
+    // each parameter's sum of this wave; D[4g + v][col]
+    float* S = lds.sums[wave];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int r = 4 * g + v;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+            const int j = mt * 16 + r;
+            if (col < kLpIn) S[kLpW1 + j * kLpIn + col] = w1[mt][v];
+            if (col == kLpIn) S[kLpB1 + j] = w1[mt][v];
+            S[kLpW2 + j * kLpHid + col] = w2[mt][0][v];
+            S[kLpW2 + j * kLpHid + 16 + col] = w2[mt][1][v];
+            if (r < kLpOut) S[kLpW3 + r * kLpHid + mt * 16 + col] = w3[mt][v];
+            float b = sb2[mt][v];  // over the 16 pixel columns
+#pragma unroll
+            for (int d = 8; d > 0; d >>= 1) b += __shfl_xor(b, d, 16);
+            if (col == 0) S[kLpB2 + j] = b;
+        }
+        float b = sb3[v];
+#pragma unroll
+        for (int d = 8; d > 0; d >>= 1) b += __shfl_xor(b, d, 16);
+        if (col == 0 && r < kLpOut) S[kLpB3 + r] = b;
+    }
+    __syncthreads();
+    for (int k = tid; k < kLpParams; k += 64 * kLpBwdWaves) {
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kLpBwdWaves; ++w) s += lds.sums[w][k];
+        partial[(size_t)blockIdx.x * kLpParams + k] = s;
     }
 }
 
-__global__ void lp_reduce_kernel(const float* __restrict__ partial, int blocks, float* __restrict__ grad) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= kLpParams) return;
+// grad += the blocks' partial sums: 16 parameters per block of 256, 16 lanes per parameter with every
+// 16th block each, added in lane order. (One lane per parameter was a chain of 240 loads: 59 us.)
+__global__ __launch_bounds__(256) void lp_reduce_kernel(const float* __restrict__ partial, int blocks,
+                                                        float* __restrict__ grad) {
+    __shared__ float part[16][17];
+    const int kl = threadIdx.x & 15, j = threadIdx.x >> 4, k = blockIdx.x * 16 + kl;
     float s = 0.0f;
-    for (int b = 0; b < blocks; ++b) s += partial[(size_t)b * kLpParams + k];
-    grad[k] += s;
+    if (k < kLpParams)
+#pragma unroll 5
+        for (int b = j; b < blocks; b += 16) s += partial[(size_t)b * kLpParams + k];
+    part[j][kl] = s;
+    __syncthreads();
+    if (j == 0 && k < kLpParams) {
+        s = 0.0f;
+        for (int q = 0; q < 16; ++q) s += part[q][kl];
+        grad[k] += s;
+    }
 }
 
 }  // namespace luxgi
@@ -505,10 +611,10 @@ extern "C" int luxgi_learned_pixel_mlp_backward(const float* params, int32_t W, 
     const long long N = (long long)W * H;
     hipStream_t st = as_stream(stream);
     float* partial = static_cast<float*>(workspace);
-    hipLaunchKernelGGL(lp_mlp_backward_kernel, dim3(kLpBwdBlocks), dim3(256), 0, st, params, N, features, gradScales,
-                       scales, partial);
+    hipLaunchKernelGGL(lp_mlp_backward_kernel, dim3(kLpBwdBlocks), dim3(64 * kLpBwdWaves), 0, st, params, N, features,
+                       gradScales, scales, partial);
     LUXGI_LAUNCH_CHECK();
-    hipLaunchKernelGGL(lp_reduce_kernel, dim3((kLpParams + 255) / 256), dim3(256), 0, st, partial, kLpBwdBlocks,
+    hipLaunchKernelGGL(lp_reduce_kernel, dim3((kLpParams + 15) / 16), dim3(256), 0, st, partial, kLpBwdBlocks,
                        gradParams);
     LUXGI_LAUNCH_CHECK();
     return LUXGI_OK;

@@ -179,6 +179,40 @@ def test_mlp_backward_matches_the_oracle_and_is_deterministic():
     assert np.allclose(got, want, rtol=2e-3, atol=1e-4 * np.abs(want).max()), np.abs(got - want).max()
 
 
+@pytest.mark.parametrize("W,H,shift", [(1, 1, 0), (5, 3, 0), (16, 1, 1), (17, 1, 0), (256, 120, 0), (31, 991, 1)])
+def test_mlp_backward_at_the_edges_of_its_pixel_tiles(W, H, shift):
+    """One pixel, one short of / one whole / one past a 16-pixel tile, and exactly / one pixel past one tile
+    per wave of the grid (240 x 8 x 16 pixels); `shift` puts the features at a 4-byte-aligned address
+    that is not 16-byte aligned. Tolerance: a hidden activation whose FP32 sum falls on the other side
+    of an FP16 rounding boundary moves its terms by 2^-11 = 4.9e-4; rtol 2e-3 covers two such layers,
+    atol 1e-4 of the largest gradient the entries that cancel."""
+    from luxgi_amd._lib import lib
+    from luxgi_amd.ddgi import ptr, stream_handle
+    rng = np.random.default_rng(W * 1000 + H)
+    p = _random_params(11)
+    N = W * H
+    f = rng.uniform(0.0, 2.0, (H, W, 12)).astype(np.float32)
+    f[..., 2:5] = rng.uniform(-1.0, 1.0, (H, W, 3))
+    buf = torch.zeros(N * 12 + 4, dtype=torch.float32, device="cuda")
+    feat = buf[shift:shift + N * 12]
+    feat.copy_(_dev(f.reshape(-1)))
+    gs = rng.normal(size=(5, H, W)).astype(np.float32)
+    pq = p.astype(np.float32).astype(np.float64)
+    scales = np.exp(rng.uniform(-1.0, 1.0, (5, H, W))).astype(np.float32)
+    ws = torch.empty(lib().luxgi_learned_pixel_mlp_backward_workspace_size(), dtype=torch.uint8, device="cuda")
+    gp = torch.zeros(abi.LEARNED_PIXEL_PARAMS, dtype=torch.float32, device="cuda")
+    # the kernel multiplies dL/ds by the scales it is given, the oracle by its own: hand it dL/do
+    own = oracle.learned_pixel_mlp(pq, f.astype(np.float64), half=True)[1]
+    print(f"mlp backward {W}x{H} shift {shift}", flush=True)
+    assert lib().luxgi_learned_pixel_mlp_backward(ptr(_dev(p.astype(np.float32))), W, H, ptr(feat), ptr(_dev(scales)),
+                                                  ptr(_dev(gs)), ptr(gp), ptr(ws), ws.numel(), stream_handle()) == 0
+    torch.cuda.synchronize()
+    want = oracle.learned_pixel_mlp_backward(pq, f.astype(np.float64),
+                                             np.moveaxis(gs.astype(np.float64) * scales, 0, -1) / own, half=True)
+    got = gp.cpu().numpy()
+    assert np.allclose(got, want, rtol=2e-3, atol=1e-4 * np.abs(want).max()), np.abs(got - want).max()
+
+
 def test_untrained_network_chain_is_the_reference_chain():
     from luxgi_amd._lib import lib
     from luxgi_amd.ddgi import ptr, stream_handle

@@ -34,32 +34,66 @@ struct AtlasGeom {
     int width, height, side, perRow;
     float invW, invH;
 };
-__device__ __forceinline__ float2 atlas_coord(f3 dir, int probe, const AtlasGeom& g) {
+// tile of a probe in the atlas: probe index over the tiles of a row. The reference's atlases hold one
+// z plane (`plane` probes wide) per row, so the tile is the probe's place in its plane and its z;
+// the division is for atlases wider than their probes need (the branch is uniform).
+__device__ __forceinline__ int2 atlas_tile(int inPlane, int z, int plane, int perRow) {
+    if (perRow == plane) return make_int2(inPlane, z);
+    const int probe = z * plane + inPlane;
+    return make_int2(probe % perRow, probe / perRow);
+}
+__device__ __forceinline__ float2 atlas_coord(f3 dir, int2 tile, const AtlasGeom& g) {
     const float2 oc = oct_encode(dir);
     const float ox = (oc.x + 1.0f) * 0.5f, oy = (oc.y + 1.0f) * 0.5f;
     const float pws = float(g.side) + 2.0f;
-    const float tlx = float(probe % g.perRow) * pws + 2.0f, tly = float(probe / g.perRow) * pws + 2.0f;
+    const float tlx = float(tile.x) * pws + 2.0f, tly = float(tile.y) * pws + 2.0f;
     return make_float2((tlx + ox * float(g.side)) * g.invW, (tly + oy * float(g.side)) * g.invH);
 }
 __host__ __device__ inline AtlasGeom atlas_geom(int width, int height, int side) {
     return AtlasGeom{width, height, side, (width - 2) / (side + 2), 1.0f / float(width), 1.0f / float(height)};
 }
 
+// i modulo n; the division only where i is outside [0, n)
 __device__ __forceinline__ int wrap_index(int i, int n) {
+    if ((unsigned)i < (unsigned)n) return i;
     const int m = i % n;
     return m < 0 ? m + n : m;
 }
 
-// texture(sampler2D, uv): bilinear, repeat addressing
+// A row of two neighbouring texels, the left one at i.
+template <class S> struct TexelPair;
+typedef float pair_f4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef uint32_t pair_u2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+template <> struct TexelPair<float> {
+    static __device__ __forceinline__ void ld2(const float* p, size_t i, float2& a, float2& b) {
+        const pair_f4_a8 v = *reinterpret_cast<const pair_f4_a8*>(p + 2 * i);
+        a = make_float2(v.x, v.y);
+        b = make_float2(v.z, v.w);
+    }
+};
+template <> struct TexelPair<__half> {
+    static __device__ __forceinline__ void ld2(const __half* p, size_t i, float2& a, float2& b) {
+        const pair_u2_a4 v = *reinterpret_cast<const pair_u2_a4*>(p + 2 * i);
+        const uint32_t x = v.x, y = v.y;
+        a = __half22float2(*reinterpret_cast<const __half2*>(&x));
+        b = __half22float2(*reinterpret_cast<const __half2*>(&y));
+    }
+};
+
+// texture(sampler2D, uv): bilinear, in a probe's bordered tile. atlas_coord keeps the footprint within
+// texels 1 .. side + 2 of the tile's row and column, and the atlas reaches past the last tile
+// (probe_atlas_geometry_valid), so the repeat addressing never wraps: the clamp only keeps a
+// footprint of non-finite coordinates inside the image. (With a modulo per index, 32 of them per
+// probe and pixel, probe sampling at 1920x1080 took 126 us against 72.)
 template <class S>
 __device__ __forceinline__ float4 bilinear4(const S* __restrict__ img, int W, int H, float u, float v) {
     const float x = u * float(W) - 0.5f, y = v * float(H) - 0.5f;
     const float fx = floorf(x), fy = floorf(y);
     const float ax = x - fx, ay = y - fy;
-    const int x0 = wrap_index(int(fx), W), x1 = wrap_index(int(fx) + 1, W);
-    const int y0 = wrap_index(int(fy), H), y1 = wrap_index(int(fy) + 1, H);
-    const float4 t00 = Texel<S>::ld4(img, (size_t)y0 * W + x0), t10 = Texel<S>::ld4(img, (size_t)y0 * W + x1);
-    const float4 t01 = Texel<S>::ld4(img, (size_t)y1 * W + x0), t11 = Texel<S>::ld4(img, (size_t)y1 * W + x1);
+    const int x0 = clampi(int(fx), 0, W - 2), y0 = clampi(int(fy), 0, H - 2);
+    const size_t e = (size_t)y0 * W + x0;
+    const float4 t00 = Texel<S>::ld4(img, e), t10 = Texel<S>::ld4(img, e + 1);
+    const float4 t01 = Texel<S>::ld4(img, e + W), t11 = Texel<S>::ld4(img, e + W + 1);
     return make_float4((t00.x * (1.0f - ax) + t10.x * ax) * (1.0f - ay) + (t01.x * (1.0f - ax) + t11.x * ax) * ay,
                        (t00.y * (1.0f - ax) + t10.y * ax) * (1.0f - ay) + (t01.y * (1.0f - ax) + t11.y * ax) * ay,
                        (t00.z * (1.0f - ax) + t10.z * ax) * (1.0f - ay) + (t01.z * (1.0f - ax) + t11.z * ax) * ay,
@@ -70,10 +104,11 @@ __device__ __forceinline__ float2 bilinear2(const S* __restrict__ img, int W, in
     const float x = u * float(W) - 0.5f, y = v * float(H) - 0.5f;
     const float fx = floorf(x), fy = floorf(y);
     const float ax = x - fx, ay = y - fy;
-    const int x0 = wrap_index(int(fx), W), x1 = wrap_index(int(fx) + 1, W);
-    const int y0 = wrap_index(int(fy), H), y1 = wrap_index(int(fy) + 1, H);
-    const float2 t00 = Texel<S>::ld2(img, (size_t)y0 * W + x0), t10 = Texel<S>::ld2(img, (size_t)y0 * W + x1);
-    const float2 t01 = Texel<S>::ld2(img, (size_t)y1 * W + x0), t11 = Texel<S>::ld2(img, (size_t)y1 * W + x1);
+    const int x0 = clampi(int(fx), 0, W - 2), y0 = clampi(int(fy), 0, H - 2);
+    const size_t e = (size_t)y0 * W + x0;
+    float2 t00, t10, t01, t11;
+    TexelPair<S>::ld2(img, e, t00, t10);
+    TexelPair<S>::ld2(img, e + W, t01, t11);
     return make_float2((t00.x * (1.0f - ax) + t10.x * ax) * (1.0f - ay) + (t01.x * (1.0f - ax) + t11.x * ax) * ay,
                        (t00.y * (1.0f - ax) + t10.y * ax) * (1.0f - ay) + (t01.y * (1.0f - ax) + t11.y * ax) * ay);
 }
@@ -112,7 +147,8 @@ __device__ f3 sample_irradiance(const LuxgiDDGIUniform& u, const AtlasGeom& irrG
         const int ox = i & 1, oy = (i >> 1) & 1, oz = (i >> 2) & 1;
         const int gx = min(bx + ox, u.probeCounts[0] - 1), gy = min(by + oy, u.probeCounts[1] - 1),
                   gz = min(bz + oz, u.probeCounts[2] - 1);
-        const int probeIdx = gx + gy * u.probeCounts[0] + gz * u.probeCounts[0] * u.probeCounts[1];
+        const int plane = u.probeCounts[0] * u.probeCounts[1], inPlane = gx + gy * u.probeCounts[0];
+        const int probeIdx = inPlane + gz * plane;
         if (rl.states && rl.states[probeIdx] != 0) continue;
         f3 probePos = mk(stp.x * float(gx) + start.x, stp.y * float(gy) + start.y, stp.z * float(gz) + start.z);
         if (rl.offsets) {
@@ -127,7 +163,7 @@ __device__ f3 sample_irradiance(const LuxgiDDGIUniform& u, const AtlasGeom& irrG
         w *= sb * sb + 0.2f;
         const f3 probeToPoint = P - probePos + vBias;
         // textureCoordFromDirection(-normalize(-probeToPoint)) == the direction of probeToPoint
-        float2 tc = atlas_coord(probeToPoint, probeIdx, depG);
+        float2 tc = atlas_coord(probeToPoint, atlas_tile(inPlane, gz, plane, depG.perRow), depG);
         const float dist = len3(probeToPoint);
         const float2 dm = bilinear2<SA>(dep, depG.width, depG.height, tc.x, tc.y);
         const float mean = dm.x;
@@ -137,7 +173,7 @@ __device__ f3 sample_irradiance(const LuxgiDDGIUniform& u, const AtlasGeom& irrG
         cheb = fmaxf(cheb * cheb * cheb, 0.0f);
         w *= (dist <= mean) ? 1.0f : cheb;
         w = fmaxf(0.000001f, w);
-        tc = atlas_coord(N, probeIdx, irrG);
+        tc = atlas_coord(N, atlas_tile(inPlane, gz, plane, irrG.perRow), irrG);
         const float4 ir = bilinear4<SA>(irr, irrG.width, irrG.height, tc.x, tc.y);
         const f3 pi = mk(fast_pow(ir.x, ge), fast_pow(ir.y, ge), fast_pow(ir.z, ge));
         if (w < 0.2f) w *= w * w * (1.0f / (0.2f * 0.2f));

@@ -132,6 +132,46 @@ def test_surface_light_matches_oracle(form):
     assert lit[drawn].mean() > 0.3
 
 
+@pytest.mark.parametrize("tile,n_lights", [(5, 1), (22, 4), (23, 5), (46, 9)])
+def test_direct_light_at_the_edges_of_the_texel_chunks_and_light_groups(tile, n_lights):
+    """Tiles of less than a wave, just under and over one 512-texel chunk, and several chunks; light
+    counts at and past the four lights whose rays are gathered together. Tolerance as in
+    test_surface_light_matches_oracle: 1% of the texels may hold a shadow ray that grazes the other way
+    with three lights, so n_lights / 300 here."""
+    from luxgi_amd.ddgi import DeviceScene
+    from luxgi_amd.surface import SurfaceCache
+    prims, sdf, mip, g, _ = _scenes.small_scene()
+    atlas = scene.build_atlas(prims, resolution=512, tile=tile, seed=3, threshold=1.05 * 2 / 64, surface_gbuffer=True)
+    ds = DeviceScene(g, sdf, mip, atlas)
+    base = _lights()
+    lights = (abi.Light * n_lights)()
+    rng = np.random.default_rng(tile)
+    for k in range(n_lights):
+        C.memmove(C.byref(lights[k]), C.byref(base[k % 3]), C.sizeof(abi.Light))
+        for j in range(3):
+            lights[k].position[j] += float(rng.uniform(-0.2, 0.2)) if k >= 3 else 0.0
+    sc = SurfaceCache(atlas, out_storage=abi.STORAGE_FP32)
+    sc.set_lights(lights)
+    cam = (0.2, 0.3, 1.8)
+    sc.light(ds, passes=abi.SURFACE_DIRECT, camera=cam, shadow_bias=0.03)
+    torch.cuda.synchronize()
+    got = sc.light_cache.cpu().numpy()
+    p = abi.SurfaceLightParams()
+    p.cameraPosition[:] = [cam[0], cam[1], cam[2], 0.03]
+    p.passes, p.numLights = abi.SURFACE_DIRECT, n_lights
+    want = oracle.surface_light(p, lights, atlas.tiles, sc.draws_host, res=512,
+                                gb_color=atlas.gb_color.astype(np.float32), gb_normal=atlas.gb_normal.astype(np.float32),
+                                gb_pbr=atlas.gb_pbr.astype(np.float32) / 255.0,
+                                gb_emissive=atlas.gb_emissive.astype(np.float32), sdf_data=g, sdf=sdf, mip=mip,
+                                sdf_res=64, mip_res=16)
+    drawn = want[..., 3] == 1.0
+    assert drawn.sum() == sc.n_draws * tile * tile
+    assert np.all(got[~drawn] == 0.0) and np.all(got[drawn][:, 3] == 1.0)
+    ok = np.all(np.abs(got[..., :3] - want[..., :3]) <= 1e-3 * np.abs(want[..., :3]) + 1e-4, axis=-1)
+    assert ok[drawn].mean() >= 1.0 - n_lights / 300.0, ok[drawn].mean()
+    assert np.abs(want[..., :3]).max() > 0.05
+
+
 def test_surface_emissive_pass_is_exact():
     from luxgi_amd.ddgi import DeviceScene
     from luxgi_amd.surface import SurfaceCache

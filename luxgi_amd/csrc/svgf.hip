@@ -36,17 +36,95 @@ struct GBuf {
 };
 
 
-// isValid (Reprojection.glsl:42-53)
-__device__ __forceinline__ bool is_valid(int hx, int hy, f3 pos, f3 prevPos, f3 n, f3 pn, float meshId,
-                                         float prevMeshId, int W, int H) {
-    if (hx < 0 || hy < 0 || hx > W - 1 || hy > H - 1) return false;
-    if (meshId != prevMeshId) return false;
-    if (fabsf(dot3(pos - prevPos, n)) > kPlaneDistance) return false;
-    const float d = fabsf(dot3(n, pn));
-    if (d * d <= kNormalDistance) return false;
-    return true;
+// isValid (Reprojection.glsl:42-53) of the taps of one pixel, with the pixel's part worked out once. The
+// reference unprojects every tap's depth pd at the pixel's history coordinate: a point
+// (a + pd b).xyz / (a + pd b).w with a and b fixed for the pixel, of which the plane test needs the
+// component along the pixel's normal only, so a tap costs two multiply-adds and a reciprocal; its
+// normal enters the angle test unnormalised, against |n|^2.
+struct TapTest {
+    f3 n;
+    float meshId, along;        // mesh id, wpos . n
+    float an, aw, bn, bw;       // a and b along n, and their w
+    bool inImage;               // the history pixel lies in the image
+};
+__device__ __forceinline__ TapTest tap_test(int hx, int hy, int W, int H, f3 wpos, f3 n, float meshId, float htx,
+                                            float hty, const float* vpi) {
+    const float4 a = mat4_mul4(vpi, make_float4(htx * 2.0f - 1.0f, hty * 2.0f - 1.0f, 0.0f, 1.0f));
+    TapTest t;
+    t.n = n;
+    t.meshId = meshId;
+    t.along = dot3(wpos, n);
+    t.an = dot3(mk(a.x, a.y, a.z), n);
+    t.aw = a.w;
+    t.bn = dot3(mk(vpi[8], vpi[9], vpi[10]), n);
+    t.bw = vpi[11];
+    t.inImage = !(hx < 0 || hy < 0 || hx > W - 1 || hy > H - 1);
+    return t;
 }
-
+// the octahedral direction before its normalisation
+__device__ __forceinline__ f3 oct_direction(float ox, float oy) {
+    f3 v = {ox, oy, 1.0f - fabsf(ox) - fabsf(oy)};
+    if (v.z < 0.0f) {
+        const float nx = (1.0f - fabsf(v.y)) * sign_not_zero(v.x), ny = (1.0f - fabsf(v.x)) * sign_not_zero(v.y);
+        v.x = nx;
+        v.y = ny;
+    }
+    return v;
+}
+struct TapTexel {
+    float2 normal;
+    float depth, meshId;
+};
+__device__ __forceinline__ TapTexel load_tap(const GBuf& prev, int x, int y, int W, int H) {
+    TapTexel t{make_float2(0.f, 0.f), 0.0f, 0.0f};
+    if (inside(x, y, W, H)) {
+        const size_t e = (size_t)y * W + x;
+        t.normal = reinterpret_cast<const float2*>(prev.normals)[2 * e];
+        t.depth = prev.depth[e];
+        t.meshId = reinterpret_cast<const float*>(prev.color)[4 * e + 3];
+    }
+    return t;
+}
+__device__ __forceinline__ bool is_valid(const TapTest& t, const TapTexel& p) {
+    if (!t.inImage || t.meshId != p.meshId) return false;
+    const float prevAlong = (t.an + p.depth * t.bn) * __builtin_amdgcn_rcpf(t.aw + p.depth * t.bw);
+    if (fabsf(t.along - prevAlong) > kPlaneDistance) return false;
+    const f3 pn = oct_direction(p.normal.x, p.normal.y);
+    const float d = dot3(t.n, pn);
+    return !(d * d <= kNormalDistance * dot3(pn, pn));
+}
+// which of the four taps at (x, y) .. (x + 1, y + 1) are valid, bit i for (i & 1, i >> 1); all loads first
+__device__ __forceinline__ int valid_taps(const TapTest& t, const GBuf& prev, int x, int y, int W, int H) {
+    TapTexel p[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = load_tap(prev, x + (i & 1), y + (i >> 1), W, H);
+    int v = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v |= is_valid(t, p[i]) ? 1 << i : 0;
+    return v;
+}
+// The 3x3 fallback's valid taps around (x, y), bit 3 (yy + 1) + xx + 1, loaded together: a loop over
+// nine tests waited for memory nine times in every wave that holds a disoccluded pixel. The second
+// form takes the four taps at (x, y) .. (x + 1, y + 1) from the first try.
+__device__ __forceinline__ int valid_taps3x3(const TapTest& t, const GBuf& prev, int x, int y, int W, int H) {
+    TapTexel p[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) p[i] = load_tap(prev, x + i % 3 - 1, y + i / 3 - 1, W, H);
+    int v = 0;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) v |= is_valid(t, p[i]) ? 1 << i : 0;
+    return v;
+}
+__device__ __forceinline__ int valid_taps3x3(const TapTest& t, int known, const GBuf& prev, int x, int y, int W, int H) {
+    constexpr int kOther[5] = {0, 1, 2, 3, 6};
+    TapTexel p[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) p[i] = load_tap(prev, x + kOther[i] % 3 - 1, y + kOther[i] / 3 - 1, W, H);
+    int v = (known & 3) << 4 | (known & 12) << 5;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) v |= is_valid(t, p[i]) ? 1 << kOther[i] : 0;
+    return v;
+}
 
 // ---------------------------------------------------------------------------
 // reflection reprojection
@@ -90,78 +168,65 @@ __device__ bool reproject_rgb(const RA& A, int cx, int cy, float depth, float ra
     }
     const int hx = int(rx), hy = int(ry);  // GLSL ivec2(): truncation
     const f3 n = oct_decode(normal.x, normal.y);
-    bool v[4];
-    bool valid = false;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int lx = hx + (i & 1), ly = hy + (i >> 1);
-        const float4 pn = fetch4(prev.normals, lx, ly, W, H);
-        const float pd = fetch1(prev.depth, lx, ly, W, H);
-        const f3 pp = world_from_depth(htx, hty, pd, A.pc.viewProjInv);
-        const float pm = fetch4(prev.color, lx, ly, W, H).w;
-        v[i] = is_valid(hx, hy, wpos, pp, n, oct_decode(pn.x, pn.y), meshId, pm, W, H);
-        valid = valid || v[i];
-    }
+    const TapTest test = tap_test(hx, hy, W, H, wpos, n, meshId, htx, hty, A.pc.viewProjInv);
     f3 col = mk(0.f, 0.f, 0.f);
     float2 mom = make_float2(0.f, 0.f);
-    if (valid) {
-        float sumw = 0.0f;
-        const float x = fractf(rx), y = fractf(ry);
-        const float w[4] = {(1.0f - x) * (1.0f - y), x * (1.0f - y), (1.0f - x) * y, x * y};
+    float len = 0.0f;
+    bool valid = false;
+    if (test.inImage) {
+        const int v = valid_taps(test, prev, hx, hy, W, H);
+        float4 c[4], m[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            c[i] = m[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             const int lx = hx + (i & 1), ly = hy + (i >> 1);
-            if (v[i]) {
-                const float4 c = fetchS4<S>(histOut, lx, ly, W, H);
-                const float4 m = fetchS4<S>(histMom, lx, ly, W, H);
-                col = col + mk(c.x, c.y, c.z) * w[i];
-                mom.x += w[i] * m.x;
-                mom.y += w[i] * m.y;
-                sumw += w[i];
+            if ((v >> i) & 1) c[i] = fetchS4<S>(histOut, lx, ly, W, H);
+            if (((v >> i) & 1) || i == 0) m[i] = fetchS4<S>(histMom, lx, ly, W, H);
+        }
+        len = m[0].z;
+        if (v) {
+            float sumw = 0.0f;
+            const float x = fractf(rx), y = fractf(ry);
+            const float w[4] = {(1.0f - x) * (1.0f - y), x * (1.0f - y), (1.0f - x) * y, x * y};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if ((v >> i) & 1) {
+                    col = col + mk(c[i].x, c[i].y, c[i].z) * w[i];
+                    mom.x += w[i] * m[i].x;
+                    mom.y += w[i] * m[i].y;
+                    sumw += w[i];
+                }
+            valid = sumw >= 0.01f;
+            if (valid) {
+                const float inv = 1.0f / sumw;
+                col = col * inv;
+                mom.x *= inv;
+                mom.y *= inv;
             }
         }
-        valid = sumw >= 0.01f;
-        if (valid) {
-            col = col * (1.0f / sumw);
-            mom.x /= sumw;
-            mom.y /= sumw;
-        } else {
+        if (!valid) {
             col = mk(0.f, 0.f, 0.f);
             mom = make_float2(0.f, 0.f);
-        }
-    }
-    if (!valid) {
-        float count = 0.0f;
-        for (int yy = -1; yy <= 1; ++yy)
-            for (int xx = -1; xx <= 1; ++xx) {
-                const int px = hx + xx, py = hy + yy;
-                const float4 pn = fetch4(prev.normals, px, py, W, H);
-                const float pd = fetch1(prev.depth, px, py, W, H);
-                const f3 pp = world_from_depth(htx, hty, pd, A.pc.viewProjInv);
-                const float pm = fetch4(prev.color, px, py, W, H).w;
-                if (is_valid(hx, hy, wpos, pp, n, oct_decode(pn.x, pn.y), meshId, pm, W, H)) {
-                    const float4 c = fetchS4<S>(histOut, px, py, W, H);
-                    const float4 m = fetchS4<S>(histMom, px, py, W, H);
-                    col = col + mk(c.x, c.y, c.z);
-                    mom.x += m.x;
-                    mom.y += m.y;
-                    count += 1.0f;
-                }
+            int near = valid_taps3x3(test, v, prev, hx, hy, W, H);
+            const float count = float(__popc(near));
+            valid = near != 0;
+            while (near) {
+                const int k = __ffs(near) - 1;
+                near &= near - 1;
+                const float4 hc4 = fetchS4<S>(histOut, hx + k % 3 - 1, hy + k / 3 - 1, W, H);
+                const float4 hm4 = fetchS4<S>(histMom, hx + k % 3 - 1, hy + k / 3 - 1, W, H);
+                col = col + mk(hc4.x, hc4.y, hc4.z);
+                mom.x += hm4.x;
+                mom.y += hm4.y;
             }
-        if (count > 0.0f) {
-            valid = true;
-            col = col * (1.0f / count);
-            mom.x /= count;
-            mom.y /= count;
+            if (valid) {
+                col = col * (1.0f / count);
+                mom.x /= count;
+                mom.y /= count;
+            }
         }
     }
-    if (valid) {
-        hl = fetchS4<S>(histMom, hx, hy, W, H).z;
-    } else {
-        col = mk(0.f, 0.f, 0.f);
-        mom = make_float2(0.f, 0.f);
-        hl = 0.0f;
-    }
+    hl = valid ? len : 0.0f;
     hc = col;
     hm = mom;
     return valid;
@@ -169,10 +234,10 @@ __device__ bool reproject_rgb(const RA& A, int cx, int cy, float depth, float ra
 
 // LDS of one reprojection block
 struct ReprojectShared {
-    // rows of 48 float3 (144 dwords, 16 banks apart): in the row sums the two rows a half-wave
-    // reads then fall in disjoint banks (a 33-wide row, 99 dwords, aliases them)
-    float3 tile[32][48];
-    float3 h1[32][16], h2[32][16];
+    // rows of 48 float3 (144 dwords, 16 banks apart): in the row sums the rows a half-wave reads then
+    // fall in disjoint banks (a 33-wide row, 99 dwords, aliases them)
+    float3 tile[32][48];       // the halo tile; then (rows 0..15) the finished sums [row][m1 | m2]
+    float3 h[2][32][16];       // row sums of c and of c * c
     int vote[4];
 };
 
@@ -185,36 +250,50 @@ __device__ __forceinline__ void reproject_block(const RA& A, const GBuf& cur, co
                                                 S* __restrict__ outMom, uint8_t* __restrict__ tileMap, int bX, int bY,
                                                 ReprojectShared& sm) {
     auto& tile = sm.tile;
-    auto& h1 = sm.h1;
-    auto& h2 = sm.h2;
     auto& vote = sm.vote;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     const int bx = bX * 16, by = bY * 16;
     const int W = A.W, H = A.H;
-    if (threadIdx.x < 4) vote[threadIdx.x] = 0;
-    for (int i = threadIdx.x; i < 32 * 32; i += 256) {
+    if (tid < 4) vote[tid] = 0;
+    for (int i = tid; i < 32 * 32; i += 256) {
         const int lx = i & 31, ly = i >> 5;
         const float4 c = fetchS4<S>(noisy, bx - 8 + lx, by - 8 + ly, W, H);
         tile[ly][lx] = make_float3(c.x, c.y, c.z);
     }
     __syncthreads();
-    for (int row = ty; row < 32; row += 16) {
-        float3 s1 = make_float3(0.f, 0.f, 0.f), s2 = make_float3(0.f, 0.f, 0.f);
-        for (int k = 0; k < 17; ++k) {
-            const float3 c = tile[row][tx + k];
+    // 17-wide sums, two neighbouring windows per lane: the 16 texels they share are read and added once
+    // (18 LDS reads for two sums instead of 34). One window per lane took 37 of the 129 us of a
+    // 1920x1080 reprojection, and its unrolled column loop 155 registers.
+    {
+        const int row = tid >> 3, g = (tid & 7) * 2;
+        float3 s1 = make_float3(0.f, 0.f, 0.f), s2 = s1;
+#pragma unroll 4
+        for (int k = 1; k < 17; ++k) {
+            const float3 c = tile[row][g + k];
             s1.x += c.x; s1.y += c.y; s1.z += c.z;
             s2.x += c.x * c.x; s2.y += c.y * c.y; s2.z += c.z * c.z;
         }
-        h1[row][tx] = s1;
-        h2[row][tx] = s2;
+        const float3 a = tile[row][g], b = tile[row][g + 17];
+        sm.h[0][row][g] = make_float3(s1.x + a.x, s1.y + a.y, s1.z + a.z);
+        sm.h[0][row][g + 1] = make_float3(s1.x + b.x, s1.y + b.y, s1.z + b.z);
+        sm.h[1][row][g] = make_float3(s2.x + a.x * a.x, s2.y + a.y * a.y, s2.z + a.z * a.z);
+        sm.h[1][row][g + 1] = make_float3(s2.x + b.x * b.x, s2.y + b.y * b.y, s2.z + b.z * b.z);
     }
     __syncthreads();
-    float3 m1 = make_float3(0.f, 0.f, 0.f), m2 = make_float3(0.f, 0.f, 0.f);
-    for (int k = 0; k < 17; ++k) {
-        const float3 a = h1[ty + k][tx], b = h2[ty + k][tx];
-        m1.x += a.x; m1.y += a.y; m1.z += a.z;
-        m2.x += b.x; m2.y += b.y; m2.z += b.z;
+    {  // columns: half the lanes sum c, half c * c (uniform per wave)
+        const int w = tid >> 7, g = ((tid >> 4) & 7) * 2;
+        float3 s = make_float3(0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int k = 1; k < 17; ++k) {
+            const float3 c = sm.h[w][g + k][tx];
+            s.x += c.x; s.y += c.y; s.z += c.z;
+        }
+        const float3 a = sm.h[w][g][tx], b = sm.h[w][g + 17][tx];
+        tile[g][w * 16 + tx] = make_float3(s.x + a.x, s.y + a.y, s.z + a.z);
+        tile[g + 1][w * 16 + tx] = make_float3(s.x + b.x, s.y + b.y, s.z + b.z);
     }
+    __syncthreads();
+    const float3 m1 = tile[ty][tx], m2 = tile[ty][16 + tx];
     const int x = bx + tx, y = by + ty;
     if (x < W && y < H) {
         const float depth = cur.depth[(size_t)y * W + x];
@@ -509,75 +588,69 @@ __device__ bool reproject_scalar(const ShadowArgs& A, int cx, int cy, float dept
     const int fxi = int(fx), fyi = int(fy);
     const float htx = tcx + mx, hty = tcy + my;
     const f3 n = oct_decode(normal.x, normal.y);
-    bool v[4];
-    bool valid = false;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int lx = fxi + (i & 1), ly = fyi + (i >> 1);
-        const float4 pn = fetch4(prev.normals, lx, ly, W, H);
-        const float pd = fetch1(prev.depth, lx, ly, W, H);
-        const f3 pp = world_from_depth(htx, hty, pd, A.pc.viewProjInv);
-        const float pm = fetch4(prev.color, lx, ly, W, H).w;
-        v[i] = is_valid(hx, hy, wpos, pp, n, oct_decode(pn.x, pn.y), meshId, pm, W, H);
-        valid = valid || v[i];
-    }
+    const TapTest test = tap_test(hx, hy, W, H, wpos, n, meshId, htx, hty, A.pc.viewProjInv);
     float col = 0.0f;
     float2 mom = make_float2(0.f, 0.f);
-    if (valid) {
-        float sumw = 0.0f;
-        const float x = fractf(fx), y = fractf(fy);
-        const float w[4] = {(1.0f - x) * (1.0f - y), x * (1.0f - y), (1.0f - x) * y, x * y};
+    float len = 0.0f;
+    bool valid = false;
+    if (test.inImage) {
+        len = fetchS4<S>(histMom, hx, hy, W, H).z;
+        const int v = valid_taps(test, prev, fxi, fyi, W, H);
+        float c[4];
+        float4 m[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            c[i] = 0.0f;
+            m[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             const int lx = fxi + (i & 1), ly = fyi + (i >> 1);
-            if (v[i]) {
-                col += w[i] * fetchS2<S>(histOut, lx, ly, W, H).x;
-                const float4 m = fetchS4<S>(histMom, lx, ly, W, H);
-                mom.x += w[i] * m.x;
-                mom.y += w[i] * m.y;
-                sumw += w[i];
+            if ((v >> i) & 1) {
+                c[i] = fetchS2<S>(histOut, lx, ly, W, H).x;
+                m[i] = fetchS4<S>(histMom, lx, ly, W, H);
             }
         }
-        valid = sumw >= 0.01f;
-        if (valid) {
-            col /= sumw;
-            mom.x /= sumw;
-            mom.y /= sumw;
-        } else {
+        if (v) {
+            float sumw = 0.0f;
+            const float x = fractf(fx), y = fractf(fy);
+            const float w[4] = {(1.0f - x) * (1.0f - y), x * (1.0f - y), (1.0f - x) * y, x * y};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if ((v >> i) & 1) {
+                    col += w[i] * c[i];
+                    mom.x += w[i] * m[i].x;
+                    mom.y += w[i] * m[i].y;
+                    sumw += w[i];
+                }
+            valid = sumw >= 0.01f;
+            if (valid) {
+                col /= sumw;
+                mom.x /= sumw;
+                mom.y /= sumw;
+            }
+        }
+        if (!valid) {
             col = 0.0f;
             mom = make_float2(0.f, 0.f);
-        }
-    }
-    if (!valid) {
-        float count = 0.0f;
-        for (int yy = -1; yy <= 1; ++yy)
-            for (int xx = -1; xx <= 1; ++xx) {
-                const int px = hx + xx, py = hy + yy;
-                const float4 pn = fetch4(prev.normals, px, py, W, H);
-                const float pd = fetch1(prev.depth, px, py, W, H);
-                const f3 pp = world_from_depth(htx, hty, pd, A.pc.viewProjInv);
-                const float pm = fetch4(prev.color, px, py, W, H).w;
-                if (is_valid(hx, hy, wpos, pp, n, oct_decode(pn.x, pn.y), meshId, pm, W, H)) {
-                    col += fetchS2<S>(histOut, px, py, W, H).x;
-                    const float4 m = fetchS4<S>(histMom, px, py, W, H);
-                    mom.x += m.x;
-                    mom.y += m.y;
-                    count += 1.0f;
-                }
+            // the fallback is centred on the history pixel, which may lie one past the taps' corner
+            int near = hx == fxi && hy == fyi ? valid_taps3x3(test, v, prev, hx, hy, W, H)
+                                              : valid_taps3x3(test, prev, hx, hy, W, H);
+            const float count = float(__popc(near));
+            valid = near != 0;
+            while (near) {
+                const int k = __ffs(near) - 1;
+                near &= near - 1;
+                col += fetchS2<S>(histOut, hx + k % 3 - 1, hy + k / 3 - 1, W, H).x;
+                const float4 hm4 = fetchS4<S>(histMom, hx + k % 3 - 1, hy + k / 3 - 1, W, H);
+                mom.x += hm4.x;
+                mom.y += hm4.y;
             }
-        if (count > 0.0f) {
-            valid = true;
-            col /= count;
-            mom.x /= count;
-            mom.y /= count;
+            if (valid) {
+                col /= count;
+                mom.x /= count;
+                mom.y /= count;
+            }
         }
     }
-    if (valid) hl = fetchS4<S>(histMom, hx, hy, W, H).z;
-    else {
-        col = 0.0f;
-        mom = make_float2(0.f, 0.f);
-        hl = 0.0f;
-    }
+    hl = valid ? len : 0.0f;
     hc = col;
     hm = mom;
     return valid;

@@ -45,12 +45,31 @@ __device__ __forceinline__ float edge_stop(float cd, float sd, float invPhiZ, f3
     return __expf(0.0f - fmaxf(wL, 0.0f) - fmaxf(wZ, 0.0f)) * wN;
 }
 
+// The same with the reference's normal exponent 32 as five squarings in line.
+__device__ __forceinline__ float edge_stop32(float cd, float sd, float invPhiZ, f3 cn, f3 sn, float cl, float sl,
+                                             float invPhiL) {
+    const float wZ = __expf(-fabsf(cd - sd) * invPhiZ);
+    float wN = clampf(dot3(cn, sn), 0.0f, 1.0f);
+    wN *= wN;
+    wN *= wN;
+    wN *= wN;
+    wN *= wN;
+    wN *= wN;
+    const float wL = fabsf(cl - sl) * invPhiL;
+    return __expf(0.0f - fmaxf(wL, 0.0f) - fmaxf(wZ, 0.0f)) * wN;
+}
+
 struct AtrousArgs {
     int W, H, tilesX, radius, stepSize;
     float phi, phiNormal, sigmaDepth, power;
     int sqNormal;            // log2(phiNormal) when it is a power of two in [1, 64], else -1
     const float* lumScale;   // optional [H][W] scale of the luminance term (learned per pixel); null = 1
 };
+
+// The reference's own filter (radius 1, normal exponent 32): the passes run their eight taps unrolled
+// and unbounded. A tap outside the image reads a zero guide, whose normal term makes its weight
+// exactly 0, so it adds nothing.
+__host__ __device__ inline bool standard_filter(const AtrousArgs& A) { return A.radius == 1 && A.sqNormal == 5; }
 
 // squarings that evaluate x^phiNormal exactly as repeated products, or -1
 __host__ __device__ inline int normal_squarings(float phiN) {
@@ -59,9 +78,22 @@ __host__ __device__ inline int normal_squarings(float phiN) {
     return -1;
 }
 
+// the octahedral direction before its normalisation
+__device__ __forceinline__ f3 oct_direction(float ox, float oy) {
+    f3 v = {ox, oy, 1.0f - fabsf(ox) - fabsf(oy)};
+    if (v.z < 0.0f) {
+        const float nx = (1.0f - fabsf(v.y)) * sign_not_zero(v.x), ny = (1.0f - fabsf(v.x)) * sign_not_zero(v.y);
+        v.x = nx;
+        v.y = ny;
+    }
+    return v;
+}
+// a texel's normal: octahedral xy only, normalised with the reciprocal square root (v_rsq_f32, within
+// 1 ulp; the square root and three divisions it stands for were a tenth of an a-trous pass)
 __device__ __forceinline__ f3 load_normal(const float4* normals, size_t q) {
-    const float2 o = reinterpret_cast<const float2*>(normals)[2 * q];  // octahedral xy only
-    return oct_decode(o.x, o.y);
+    const float2 o = reinterpret_cast<const float2*>(normals)[2 * q];
+    const f3 v = oct_direction(o.x, o.y);
+    return v * __builtin_amdgcn_rsqf(dot3(v, v));
 }
 __device__ __forceinline__ float load_linear_depth(const float4* pbr, size_t q) {
     return reinterpret_cast<const float*>(pbr)[4 * q + 3];

@@ -270,6 +270,37 @@ def test_atrous_footprints_lds_and_direct(radius, step):
     np.testing.assert_allclose(sout.cpu().numpy(), sref, rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("W,H", [(1, 1), (7, 3), (16, 16), (33, 17)])
+@pytest.mark.parametrize("step,phi_normal", [(1, 32.0), (2, 32.0), (8, 32.0), (16, 32.0), (1, 16.0), (16, 5.5)])
+def test_atrous_at_image_edges_for_the_unrolled_and_the_general_filter(W, H, step, phi_normal):
+    """Radius 1 with the normal exponent 32 runs the unrolled filter, whose taps outside the image weigh
+    nothing; other exponents run the general loop. Images of one pixel, smaller than the step, one
+    block, and one pixel past it in both directions. Tolerances of the footprint test above."""
+    from luxgi_amd import _lib
+    from luxgi_amd.ddgi import ptr, stream_handle
+    from luxgi_amd.svgf import gbuffer_struct
+    g, *_ = _svgf_inputs.make_pair(W, H, 3)
+    dg = _dev(g)
+    rng = np.random.default_rng(W * 100 + H + step)
+    tiles = np.ones(_lib.lib().luxgi_svgf_tile_count(W, H), np.uint8)
+    ttiles = torch.from_numpy(tiles).cuda()
+    x4 = rng.uniform(0, 1.5, (H, W, 4)).astype(np.float32)
+    ap = abi.ReflectionAtrousParams(1, step, 10.0, phi_normal, 1.0, 1)
+    tin, tout = torch.from_numpy(x4).cuda(), torch.zeros((H, W, 4), device="cuda")
+    assert _lib.lib().luxgi_svgf_reflection_atrous(C.byref(ap), W, H, 0, C.byref(gbuffer_struct(dg)), ptr(ttiles),
+                                                   ptr(tin), ptr(tout), None, stream_handle()) == 0
+    sp = abi.ShadowAtrousParams(1, step, 10.0, phi_normal, 1.0, 1.2, 0.1, 1000.0)
+    x2 = np.ascontiguousarray(x4[..., :2] / 1.5)
+    sin, sout = torch.from_numpy(x2).cuda(), torch.ones((H, W, 2), device="cuda")
+    assert _lib.lib().luxgi_svgf_shadow_atrous(C.byref(sp), W, H, 0, C.byref(gbuffer_struct(dg)), ptr(ttiles),
+                                               ptr(sin), ptr(sout), None, stream_handle()) == 0
+    torch.cuda.synchronize()
+    ref = oracle.reflection_atrous(ap, W, H, g["normals"], g["pbr"], tiles, x4)
+    np.testing.assert_allclose(tout.cpu().numpy(), ref, rtol=1e-4, atol=1e-5)
+    sref = oracle.shadow_atrous(sp, W, H, g["normals"], g["pbr"], tiles, x2)
+    np.testing.assert_allclose(sout.cpu().numpy(), sref, rtol=1e-4, atol=1e-5)
+
+
 def test_atrous_rejects_bad_steps():
     from luxgi_amd import _lib
     from luxgi_amd.ddgi import ptr, stream_handle

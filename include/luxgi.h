@@ -123,8 +123,8 @@ typedef struct LuxgiTraceParams {
     /* --- extensions (defaults reproduce the reference) --- */
     int32_t  maxSteps;      /* per-cascade step cap; reference = 250 (SDFCommon.glsl:143) */
     float    hitEpsilon;    /* 0 = reference thickness test (SDFCommon.glsl:166-167); >0 = fixed eps */
-    int32_t  shadeOrder;    /* 0 = shade hit rays grouped by surface-atlas chunk (counting sort in the
-                               workspace), 1 = in ray order; the outputs are identical */
+    int32_t  shadeOrder;    /* 0 or 1. Both shade in ray order, a wave's hits grouped as it goes (0 once sorted
+                               the hits by surface-atlas chunk); the outputs are identical */
     int32_t  pad1;
     float    skyColor[4];   /* sky radiance when no cubemap is bound (reference binds a unit cube) */
     const float* deviceOrientation; /* optional device array of 16 floats (column-major): read in place of
@@ -255,7 +255,7 @@ int luxgi_ddgi_fill_atlas_sizes(LuxgiDDGIUniform* uniform);
 
 /* Workspace bytes needed by luxgi_ddgi_trace_sdf for the probe grid of `uniform`
  * and `objectCapacity` atlas objects (per-object inverse transforms and the
- * 24-byte per-ray march records that the shading kernel consumes). */
+ * 17-byte per-ray march records that the shading kernel consumes). */
 size_t luxgi_ddgi_trace_workspace_size(const LuxgiDDGIUniform* uniform, int32_t objectCapacity);
 
 /* GISDFRays.comp (Shaders/DDGI/GISDFRays.comp:63-128): probe ray generation,

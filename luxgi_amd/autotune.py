@@ -106,8 +106,8 @@ def tune_svgf_batch(batch, tuner=None, check=True):
 
 
 def tune_trace_shade_order(volume, scene, params, tuner=None):
-    """Chooses the trace's shading order (0: hits sorted by surface-atlas chunk, 1: ray order) for a
-    DDGIVolume and scene; both give identical ray data. Sets params.shadeOrder and returns it."""
+    """Times the trace's two shadeOrder values for a DDGIVolume and scene (both shade in ray order and give
+    identical ray data), sets params.shadeOrder to the faster and returns it."""
     tuner = tuner or Autotuner()
     u = volume.u
     sig = f"{u.probeCounts[0]}x{u.probeCounts[1]}x{u.probeCounts[2]}x{u.raysPerProbe}|{scene.n_objects}"

@@ -56,10 +56,7 @@ __device__ __forceinline__ void gather_footprint(int res, float u, float v, size
     float x = u * float(res) - 0.5f, y = v * float(res) - 0.5f;
     int i0 = int(floorf(x)), j0 = int(floorf(y));
     int i1 = i0 + 1, j1 = j0 + 1;
-    auto wrap = [res](int i) {
-        int m = i % res;
-        return m < 0 ? m + res : m;
-    };
+    auto wrap = [res](int i) { return wrap_index(i, res); };
     i0 = wrap(i0); i1 = wrap(i1); j0 = wrap(j0); j1 = wrap(j1);
     if constexpr (std::is_same<SC, PackedAtlas>::value) {
         idx[0] = atlas_block_index(i0, j1, res);
@@ -91,20 +88,24 @@ __device__ float4 sample_tile(const LuxgiSurfaceAtlasData& ad, const LuxgiAtlasT
     for (int k = 0; k < 16; ++k) tm[k] = tp->transform[k];
     const float4 ob = *reinterpret_cast<const float4*>(tp->objectBounds);
     const float4 ex = *reinterpret_cast<const float4*>(tp->extends);
-    f3 n = normalize3(mat4_mul(tm, ln, 1.0f));
+    // divisions by the tile's sizes and by constants are multiplications by reciprocals (v_rcp_f32, within
+    // 1 ulp), the normal is normalised with the reciprocal square root: they only scale weights
+    const f3 n = fast_normalize(mat4_mul(tm, ln, 1.0f));
     float nw = clampf(n.z, 0.0f, 1.0f);
-    nw = (nw - 0.05f) / (1.0f - 0.05f);
+    nw = (nw - 0.05f) * (1.0f / (1.0f - 0.05f));
     if (nw <= 0.0f) return make_float4(0.f, 0.f, 0.f, 0.f);
-    f3 t = mat4_mul(tm, lp, 1.0f);
-    const float tileDepth = t.z / ob.z;
-    const float tu = clampf(t.x / ob.x + 0.5f, 0.0f, 1.0f), tv = clampf(t.y / ob.y + 0.5f, 0.0f, 1.0f);
+    const f3 t = mat4_mul(tm, lp, 1.0f);
+    const float invZ = __builtin_amdgcn_rcpf(ob.z);
+    const float tileDepth = t.z * invZ;
+    const float tu = clampf(t.x * __builtin_amdgcn_rcpf(ob.x) + 0.5f, 0.0f, 1.0f);
+    const float tv = clampf(t.y * __builtin_amdgcn_rcpf(ob.y) + 0.5f, 0.0f, 1.0f);
     const float au = tu * ex.z + ex.x, av = tv * ex.w + ex.y;
     const float bx = fractf(au * float(ad.resolution) + 0.5f), by = fractf(av * float(ad.resolution) + 0.5f);
     float bw[4] = {(1.0f - bx) * by, bx * by, bx * (1.0f - by), (1.0f - bx) * (1.0f - by)};
     size_t idx[4];
     gather_footprint<SC>((int)ad.resolution, au, av, idx);
     if (COUNT) c.tiles++;
-    const float thr = 2.0f * threshold / ob.z;
+    const float thr = 2.0f * threshold * invZ, invThr = 2.0f * __builtin_amdgcn_rcpf(thr);
     float vis[4];
     uint2 packed[4];
     if constexpr (kPacked) {
@@ -116,7 +117,7 @@ __device__ float4 sample_tile(const LuxgiSurfaceAtlasData& ad, const LuxgiAtlasT
         float tz;
         if constexpr (kPacked) tz = __uint_as_float(packed[i].y);
         else tz = depth[idx[i]];
-        vis[i] = 1.0f - clampf((fabsf(tileDepth - tz) - thr) / (0.5f * thr), 0.0f, 1.0f);
+        vis[i] = 1.0f - clampf((fabsf(tileDepth - tz) - thr) * invThr, 0.0f, 1.0f);
         if (tz >= 1.0f) vis[i] = 0.0f;
     }
     float sw = vis[0] * bw[0] + vis[1] * bw[1] + vis[2] * bw[2] + vis[3] * bw[3];
@@ -136,6 +137,90 @@ __device__ float4 sample_tile(const LuxgiSurfaceAtlasData& ad, const LuxgiAtlasT
     return make_float4(r * sw, g * sw, b * sw, sw);
 }
 
+// chunk of a world position (AtlasCommon.glsl:118-122)
+__device__ __forceinline__ int atlas_chunk(const LuxgiSurfaceAtlasData& ad, f3 wp) {
+    int cc[3];
+    const float pc[3] = {wp.x, wp.y, wp.z};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) cc[i] = clampi(int(floorf(pc[i] / ad.chunkSize + float(kChunksRes) * 0.5f)), 0, kChunksRes - 1);
+    return cc[2] * kChunksRes * kChunksRes + cc[1] * kChunksRes + cc[0];
+}
+
+// LDS written by some lanes of a wave and read by others of the same wave: the LDS serves a wave's
+// accesses in order, so only the compiler has to be held
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// sampleGlobalSurfaceAtlas (AtlasCommon.glsl:115-157) by groups of eight lanes: every lane of a group
+// passes its group's point, normal, threshold and object list (`list`: the first id's place in
+// `culled`, `count` ids, 0 for a group without a point), and all get the result. The whole wave
+// calls it. The eight lanes test eight objects of the list together; each object that holds the point
+// is then sampled with one tile per lane. Each lane sums its tile over the objects, in list order,
+// and the lanes' sums are added pairwise.
+template <class SC, bool COUNT>
+__device__ __forceinline__ float4 sample_atlas_group(const LuxgiSurfaceAtlasData& ad, const uint32_t* __restrict__ culled,
+                                                     const LuxgiAtlasObject* __restrict__ objects,
+                                                     const float* __restrict__ objInv,
+                                                     const LuxgiAtlasTile* __restrict__ tiles,
+                                                     const SC* __restrict__ color, const float* __restrict__ depth,
+                                                     f3 wp, f3 wn, float threshold, uint32_t list, uint32_t count,
+                                                     Counts& c) {
+    const int lane = threadIdx.x & 63, t = lane & 7, base = lane & 56;
+    float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t o0 = 0; __any(o0 < count); o0 += 8) {
+        bool holds = false;
+        uint32_t id = 0;
+        f3 lp = mk(0.f, 0.f, 0.f), ln = lp;
+        if (o0 + t < count) {
+            id = culled[list + o0 + t];
+            const LuxgiAtlasObject* o = objects + id;
+            if (COUNT) c.objects++;
+            const float4 bs = *reinterpret_cast<const float4*>(o->objectBounds);
+            const float4 e = *reinterpret_cast<const float4*>(o->extends);
+            const float* inv = objInv + (size_t)id * 16;
+            float m[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) m[k] = inv[k];
+            if (!(len3(mk(bs.x, bs.y, bs.z) - wp) > bs.w)) {
+                const float4 l4 = mat4_mul4(m, make_float4(wp.x, wp.y, wp.z, 1.0f));
+                lp = mk(l4.x, l4.y, l4.z);
+                holds = !(fabsf(lp.x) > e.x + threshold || fabsf(lp.y) > e.y + threshold || fabsf(lp.z) > e.z + threshold);
+                ln = mk(m[0] * wn.x + m[4] * wn.y + m[8] * wn.z, m[1] * wn.x + m[5] * wn.y + m[9] * wn.z,
+                        m[2] * wn.x + m[6] * wn.y + m[10] * wn.z);
+                ln = fast_normalize(ln);
+            }
+        }
+        uint32_t left = (uint32_t)(__ballot(holds) >> base) & 0xffu;  // the group's objects, in list order
+        while (__any(left != 0)) {
+            const int src = base + (left ? __ffs(left) - 1 : 0);
+            const uint32_t oid = (uint32_t)__shfl((int)id, src);
+            const f3 p = mk(__shfl(lp.x, src), __shfl(lp.y, src), __shfl(lp.z, src));
+            const f3 n = mk(__shfl(ln.x, src), __shfl(ln.y, src), __shfl(ln.z, src));
+            const uint32_t to = left && t < 6 ? objects[oid].tileOffset[t] : 0u;
+            left &= left - 1;
+            if (to != 0) {
+                const float4 s = sample_tile<SC, COUNT>(ad, tiles + to, color, depth, p, n, threshold, c);
+                res.x += s.x;
+                res.y += s.y;
+                res.z += s.z;
+                res.w += s.w;
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) {
+        res.x += __shfl_xor(res.x, d);
+        res.y += __shfl_xor(res.y, d);
+        res.z += __shfl_xor(res.z, d);
+        res.w += __shfl_xor(res.w, d);
+    }
+    const float a = 1.0f / fmaxf(res.w, 0.0001f);
+    return make_float4(res.x * a, res.y * a, res.z * a, res.w);
+}
+
 // sampleGlobalSurfaceAtlas (AtlasCommon.glsl:115-157), debug = false: (rgb / max(a, 1e-4), a) with a
 // the summed tile weights, (0, 0, 0, 0) when the chunk has no list
 template <class SC, bool COUNT>
@@ -145,11 +230,7 @@ __device__ float4 sample_atlas(const LuxgiSurfaceAtlasData& ad, const uint32_t* 
                                const SC* __restrict__ color, const float* __restrict__ depth, f3 wp, f3 wn,
                                float threshold, Counts& c) {
     float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
-    int cc[3];
-    const float pc[3] = {wp.x, wp.y, wp.z};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) cc[i] = clampi(int(floorf(pc[i] / ad.chunkSize + float(kChunksRes) * 0.5f)), 0, kChunksRes - 1);
-    uint32_t start = chunks[cc[2] * kChunksRes * kChunksRes + cc[1] * kChunksRes + cc[0]];
+    uint32_t start = chunks[atlas_chunk(ad, wp)];
     if (start == 0) return make_float4(0.f, 0.f, 0.f, 0.f);
     const uint32_t count = culled[start];
     if (count > ad.objectsCount) return make_float4(0.f, 0.f, 0.f, 0.f);
@@ -170,7 +251,7 @@ __device__ float4 sample_atlas(const LuxgiSurfaceAtlasData& ad, const uint32_t* 
         if (fabsf(lp.x) > e.x + threshold || fabsf(lp.y) > e.y + threshold || fabsf(lp.z) > e.z + threshold) continue;
         f3 ln = mk(m[0] * wn.x + m[4] * wn.y + m[8] * wn.z, m[1] * wn.x + m[5] * wn.y + m[9] * wn.z,
                    m[2] * wn.x + m[6] * wn.y + m[10] * wn.z);
-        ln = normalize3(ln);
+        ln = fast_normalize(ln);
         for (int t = 0; t < 6; ++t) {
             const uint32_t to = o->tileOffset[t];
             if (to != 0) {

@@ -12,7 +12,10 @@
 // each candidate object's transform per hit (AtlasCommon.glsl:134); here the
 // inverses are computed once per call into the workspace (trace_prepare_kernel).
 // The march (march_kernel) and the per-hit work (shade_kernel) are separate
-// launches, so the march loop carries only the registers it needs.
+// launches, so the march loop carries only the registers it needs. The march
+// stores everything that needs no atlas lookup: the final results of misses and
+// inside hits, and the direction and distance of the front hits. The shade adds
+// the front hits' radiance.
 #include "atlas_sample.hpp"
 #include "sdf_trace.hpp"
 
@@ -55,35 +58,11 @@ struct TraceArgs {
     int maxSteps, P, R, rayWidth;
     float hitEps;
     int fineLayout;                // LuxgiLayout of the fine volume (the kernels' template argument)
-    int sortHits;                  // shade the hit rays grouped by surface-atlas chunk
     LuxgiTraceVolume vol;          // the volume of a single-volume call
     const LuxgiTraceVolume* vols;  // the volumes of a batched call (device memory), their count
     int nVols;                     // and the total of their rays
     long long totalRays;
 };
-
-constexpr int kChunkBins = kChunksRes * kChunksRes * kChunksRes;
-constexpr uint32_t kNoChunk = 0xffffffffu;  // misses and inside hits: no atlas lookup
-
-// Adds the wave's active lanes to counters[key] with one atomic per distinct key and returns each
-// lane's slot (the counter's old value + the lane's rank among the lanes with its key). Called by
-// all 64 lanes of the wave together.
-__device__ __forceinline__ uint32_t wave_aggregated_add(uint32_t* __restrict__ counters, uint32_t key, bool active) {
-    const int lane = threadIdx.x & 63;
-    unsigned long long todo = __ballot(active);
-    uint32_t slot = 0;
-    while (todo) {
-        const int leader = __ffsll((long long)todo) - 1;
-        const uint32_t lk = (uint32_t)__shfl((int)key, leader);
-        const unsigned long long peers = todo & __ballot(key == lk);
-        uint32_t base = 0;
-        if (lane == leader) base = atomicAdd(&counters[lk], (uint32_t)__popcll(peers));
-        base = (uint32_t)__shfl((int)base, leader);
-        if ((peers >> lane) & 1ull) slot = base + (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
-        todo &= ~peers;
-    }
-    return slot;
-}
 
 // ---------------------------------------------------------------------------
 // March (tracyGlobalSDF, SDFCommon.glsl:98-194): one lane per ray, the 64 lanes
@@ -91,8 +70,8 @@ __device__ __forceinline__ uint32_t wave_aggregated_add(uint32_t* __restrict__ c
 // the dispatcher deals blocks to the 8 XCDs round-robin, so block b runs on XCD
 // b % 8; the mapping gives each XCD a contiguous range of rays (a slab of
 // probes) that it walks in order, which keeps the SDF lines its rays touch in
-// its own L2. The hit record (hitTime, texture UV of the hit step, hit SDF,
-// cascade) goes to the workspace and shade_kernel turns it into the outputs.
+// its own L2. A front hit's record (hitTime, texture UV of the hit step; cascade)
+// goes to the workspace for shade_kernel.
 // ---------------------------------------------------------------------------
 
 __device__ __forceinline__ void ray_setup(const TraceArgs& A, const LuxgiTraceVolume& v, int probe, int ray,
@@ -167,16 +146,6 @@ __device__ __forceinline__ void store_nonhit(const TraceArgs& A, const TraceScen
     Texel<SR>::st4(outRad, e, rad);
     Texel<SR>::st4(outDD, e, make_float4(dir.x, dir.y, dir.z, kWorldSize));
     if (flags) flags[e] = inside ? 2 : 0;
-}
-
-// Slot of a hit in its chunk's run of the sorted order: one atomic per lane, or one per distinct
-// chunk of the wave.
-__device__ __forceinline__ uint32_t hist_add(uint32_t* __restrict__ bins, uint32_t key, bool active) {
-#if LUXGI_HIST_PER_LANE
-    return active ? atomicAdd(&bins[key], 1u) : 0u;
-#else
-    return wave_aggregated_add(bins, key, active);
-#endif
 }
 
 // State of one ray's sphere trace (SDFCommon.glsl:98-171), advanced one step at a time.
@@ -287,45 +256,41 @@ __device__ __forceinline__ bool march_step(const TraceArgs& A, const TraceScene&
     return false;
 }
 
-// What a finished ray leaves: its hit record and, with the hit sort, either its final result (no
-// atlas lookup: miss or inside hit) or its atlas chunk (returned; kNoChunk otherwise).
+// What a finished ray leaves: a front hit its direction, distance and flag (GISDFRays.comp:121-127) and
+// its record for the shade; any other ray its final result and a record without a hit. `end` is the
+// end of the march: (hit time or < 0, texture UV), `rb` (distance, cascade).
 template <class SR>
-__device__ __forceinline__ uint32_t march_finish(const TraceArgs& A, const TraceScene& S, const LuxgiTraceVolume& v, const MarchRay& r,
-                                                 float4 ra, float2 rb, int probe, int ray, size_t rid,
-                                                 float4* __restrict__ recA, float2* __restrict__ recB,
-                                                 const float* __restrict__ skyFaces) {
-    recA[rid] = ra;
-    recB[rid] = rb;
-    uint32_t key = kNoChunk;
-    if (A.sortHits) {
-        const bool inside = ra.x >= 0.0f && rb.x <= 0.0f && ra.x <= S.g.cascadeVoxelSize[0];
-        if (ra.x >= 0.0f && !inside) {  // atlas chunk of a front hit (the lookup of sample_atlas)
-            const f3 hp = r.o + r.d * ra.x;
-            const float pc[3] = {hp.x, hp.y, hp.z};
-            int cc[3];
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                cc[i] = clampi(int(floorf(pc[i] / S.ad.chunkSize + float(kChunksRes) * 0.5f)), 0, kChunksRes - 1);
-            key = (uint32_t)((cc[2] * kChunksRes + cc[1]) * kChunksRes + cc[0]);
-        } else {
-            store_nonhit<SR>(A, S, skyFaces, static_cast<SR*>(v.rays.radiance), static_cast<SR*>(v.rays.directionDistance),
-                             v.rayFlags, (size_t)probe * v.rays.width + ray, r.d, inside);
-        }
+__device__ __forceinline__ void march_finish(const TraceArgs& A, const TraceScene& S, const LuxgiTraceVolume& v,
+                                             const MarchRay& r, float4 end, float2 rb, int probe, int ray, size_t rid,
+                                             float4* __restrict__ recA, uint8_t* __restrict__ recC) {
+    SR* outRad = static_cast<SR*>(v.rays.radiance);
+    SR* outDD = static_cast<SR*>(v.rays.directionDistance);
+    const size_t e = (size_t)probe * v.rays.width + ray;
+    const bool inside = end.x >= 0.0f && rb.x <= 0.0f && end.x <= S.g.cascadeVoxelSize[0];
+    if (end.x >= 0.0f && !inside) {
+        const int cas = int(rb.y);
+        const float dist = fmaxf(end.x + S.g.cascadeVoxelSize[cas] * 0.5f, 0.0f);
+        Texel<SR>::st4(outDD, e, make_float4(r.d.x, r.d.y, r.d.z, dist));
+        if (v.rayFlags) v.rayFlags[e] = 1;
+        recC[rid] = (uint8_t)cas;
+    } else {
+        store_nonhit<SR>(A, S, S.skyFaces, outRad, outDD, v.rayFlags, e, r.d, inside);
+        end.x = -1.0f;
     }
-    return key;
+    recA[rid] = end;
 }
 
 __device__ __forceinline__ float trace_max_distance(const TraceArgs& A, const TraceScene& S) {
     return fminf(kWorldSize, S.g.cascadePosDistance[(int)S.g.cascadesCount - 1][3] * 2.0f);
 }
 
-// The sphere trace of one ray (SDFCommon.glsl:98-171) through its cascades; returns its hit chunk
-// (kNoChunk when it needs no atlas lookup).
+// The sphere trace of one ray (SDFCommon.glsl:98-171) through its cascades.
 template <class SS, class SR, bool COUNT, int FL>
-__device__ __forceinline__ uint32_t march_ray(const TraceArgs& A, const TraceScene& S, const LuxgiTraceVolume& v,
-                                              int probe, int ray, size_t rid, float4* __restrict__ recA,
-                                              float2* __restrict__ recB, unsigned long long& cMip,
-                                              unsigned long long& cFine, unsigned long long& cSteps) {
+__device__ __forceinline__ void march_ray(const TraceArgs& A, const TraceScene& S, const LuxgiTraceVolume& v,
+                                          int probe, int ray, size_t rid, float4* __restrict__ recA,
+                                          uint8_t* __restrict__ recC, unsigned long long& cMip,
+                                          unsigned long long& cFine, unsigned long long& cSteps,
+                                          unsigned long long& cHits) {
     const SS* sdf = static_cast<const SS*>(S.sdf);
     const SS* mip = static_cast<const SS*>(S.mip);
     const int C = (int)S.g.cascadesCount;
@@ -346,7 +311,8 @@ __device__ __forceinline__ uint32_t march_ray(const TraceArgs& A, const TraceSce
         if (hit || ++r.cas >= C) break;
         march_enter(A, S, r, traceMax);
     }
-    return march_finish<SR>(A, S, v, r, ra, rb, probe, ray, rid, recA, recB, S.skyFaces);
+    if (COUNT && ra.x >= 0.0f) cHits++;
+    march_finish<SR>(A, S, v, r, ra, rb, probe, ray, rid, recA, recC);
 }
 
 // The volume of flat ray `gid` of a batch (MODE 1: one scene, MODE 2: a scene per volume). In MODE
@@ -368,211 +334,175 @@ __device__ __forceinline__ long long volume_rays(const LuxgiTraceVolume& v) {
            v.uniform.raysPerProbe;
 }
 
-// Sphere trace of one ray per lane. Writes the hit record; with the hit sort it also writes the
-// final result of the rays without an atlas lookup and the (chunk, slot) of the others. MODE 0 (one
-// volume): 64 rays of one probe per wave (rays padded to a multiple of 64 per probe). MODE 1 and 2
-// (batches over one scene / a scene per volume): the flat ray list of all volumes, each ray finding
-// its volume by rayStart; a ray past its volume's rays (padding, or a stale totalRays) does nothing.
-template <class SS, class SR, bool COUNT, int FL, int MODE>
-__global__ __launch_bounds__(256) void march_kernel(TraceArgs A, float4* __restrict__ recA, float2* __restrict__ recB,
-                                                    uint2* __restrict__ hitKeys, uint32_t* __restrict__ bins,
-                                                    unsigned long long* __restrict__ counters) {
-    const long long gb = xcd_block(blockIdx.x, gridDim.x);
-    const long long gid = gb * blockDim.x + threadIdx.x;
-    unsigned long long cMip = 0, cFine = 0, cSteps = 0;
-    uint32_t key = kNoChunk;
-    bool valid;
-    size_t rid;
-    if constexpr (MODE != 0) {
-        valid = gid < A.totalRays;
-        rid = (size_t)gid;
-        if (MODE == 2 || valid) {
-            const LuxgiTraceVolume& v = A.vols[batch_volume<MODE>(A, gid)];
-            const int R = v.uniform.raysPerProbe;
-            const long long local = gid - v.rayStart;
-            valid = valid && local >= 0 && local < volume_rays(v);
-            if (valid)
-                key = march_ray<SS, SR, COUNT, FL>(A, MODE == 2 ? A.scenes[v.scene] : A.scene, v, int(local / R),
-                                                   int(local % R), rid, recA, recB, cMip, cFine, cSteps);
-        }
-    } else {
+// The ray of flat lane `gid`: false past the rays. MODE 0 (one volume): 64 rays of one probe per wave
+// (rays padded to a multiple of 64 per probe). MODE 1 and 2 (batches over one scene / a scene per
+// volume): the flat ray list of all volumes, each ray finding its volume by rayStart; a ray past its
+// volume's rays (padding, or a stale totalRays) does nothing.
+template <int MODE>
+__device__ __forceinline__ bool find_ray(const TraceArgs& A, long long gid, const LuxgiTraceVolume*& v, int& probe,
+                                         int& ray, size_t& rid) {
+    if constexpr (MODE == 0) {
         const int Rp = (A.R + 63) & ~63;
-        const int probe = int(gid / Rp), ray = int(gid % Rp);
-        valid = probe < A.P && ray < A.R;
+        v = &A.vol;
+        probe = int(gid / Rp);
+        ray = int(gid % Rp);
         rid = (size_t)probe * A.R + ray;
-        if (valid) key = march_ray<SS, SR, COUNT, FL>(A, A.scene, A.vol, probe, ray, rid, recA, recB, cMip, cFine, cSteps);
+        return probe < A.P && ray < A.R;
+    } else {
+        v = &A.vols[batch_volume<MODE>(A, gid)];
+        const int R = v->uniform.raysPerProbe;
+        const long long local = gid - v->rayStart;
+        probe = int(local / R);
+        ray = int(local % R);
+        rid = (size_t)gid;
+        return gid < A.totalRays && local >= 0 && local < volume_rays(*v);
     }
-    if (A.sortHits) {  // chunk histogram; each hit keeps its slot within its chunk
-        const uint32_t slot = hist_add(bins, key, key != kNoChunk);
-        if (valid) hitKeys[rid] = make_uint2(key, slot);
-    }
+}
+
+// Sphere trace of one ray per lane.
+template <class SS, class SR, bool COUNT, int FL, int MODE>
+__global__ __launch_bounds__(256) void march_kernel(TraceArgs A, float4* __restrict__ recA, uint8_t* __restrict__ recC,
+                                                    unsigned long long* __restrict__ counters) {
+    const long long gid = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    unsigned long long cMip = 0, cFine = 0, cSteps = 0, cHits = 0;
+    const LuxgiTraceVolume* v;
+    int probe, ray;
+    size_t rid;
+    if (find_ray<MODE>(A, gid, v, probe, ray, rid))
+        march_ray<SS, SR, COUNT, FL>(A, MODE == 2 ? A.scenes[v->scene] : A.scene, *v, probe, ray, rid, recA, recC, cMip,
+                                     cFine, cSteps, cHits);
     if (COUNT) {
-        __shared__ unsigned long long sc[3];
-        if (threadIdx.x < 3) sc[threadIdx.x] = 0;
+        __shared__ unsigned long long sc[4];
+        if (threadIdx.x < 4) sc[threadIdx.x] = 0;
         __syncthreads();
         atomicAdd(&sc[0], cMip);
         atomicAdd(&sc[1], cFine);
         atomicAdd(&sc[2], cSteps);
+        atomicAdd(&sc[3], cHits);
         __syncthreads();
         if (threadIdx.x == 0) {
             atomicAdd(&counters[0], sc[0]);
             atomicAdd(&counters[1], sc[1]);
             atomicAdd(&counters[6], sc[2]);
+            atomicAdd(&counters[7], sc[3]);
         }
     }
 }
 
-// Normal, surface-atlas lookup and ray-result encode (SDFCommon.glsl:172-184,
-// GISDFRays.comp:89-127) for one ray.
-template <class SS, class SC, class SR, bool COUNT>
-__device__ __forceinline__ void shade_ray(const TraceArgs& A, const TraceScene& S, const LuxgiTraceVolume& v, int probe,
-                                          int ray, size_t rid, const float* __restrict__ objInvBase,
-                                          const float4* __restrict__ recA, const float2* __restrict__ recB, Counts& c) {
-    const SS* sdf = static_cast<const SS*>(S.sdf);
-    const float* skyFaces = S.skyFaces;
-    SR* outRad = static_cast<SR*>(v.rays.radiance);
-    SR* outDD = static_cast<SR*>(v.rays.directionDistance);
-    uint8_t* flags = v.rayFlags;
-    f3 origin, dir;
-    ray_setup(A, v, probe, ray, origin, dir);
-    const float4 ra = recA[rid];
-    const float hitTime = ra.x;
-    const size_t e = (size_t)probe * v.rays.width + ray;
-    if (hitTime >= 0.0f) {
-        const float2 rb = recB[rid];
-        const float hitSdf = rb.x;
-        const int hitCascade = int(rb.y);
-        if (COUNT) c.hits++;
-        if (hitSdf <= 0.0f && hitTime <= S.g.cascadeVoxelSize[0]) {
-            store_nonhit<SR>(A, S, skyFaces, outRad, outDD, flags, e, dir, true);
-        } else {
-            const int C = (int)S.g.cascadesCount;
-            const int texW = S.res * C;
-            const float o = 1.0f / S.g.resolution;
-            const float tx = ra.y, uy = ra.z, uz = ra.w;
-            auto nl = [&](float u_, float v_, float w_) {
-                if (S.refine) return refine_lookup(A, S, texW, S.res, S.res, u_, v_, w_);
-                if (A.fineLayout == LUXGI_LAYOUT_BRICK4)
-                    return sample3d_brick4<SS>(sdf, texW, S.res, S.res, u_, v_, w_, S.brickScale);
-                if (A.fineLayout == LUXGI_LAYOUT_CELL8) return sample3d_cell8<SS>(sdf, texW, S.res, S.res, u_, v_, w_);
-                return sample_volume<SS>(sdf, texW, S.res, S.res, u_, v_, w_);
-            };
-            const float xp = nl(tx + o, uy, uz), xn = nl(tx - o, uy, uz);
-            const float yp = nl(tx, uy + o, uz), yn = nl(tx, uy - o, uz);
-            const float zp = nl(tx, uy, uz + o), zn = nl(tx, uy, uz - o);
-            const f3 n = normalize3(mk(xp - xn, yp - yn, zp - zn));
-            if (COUNT) c.normals++;
-            const f3 hp = origin + dir * hitTime;
-            const float thr = S.g.cascadeVoxelSize[hitCascade] * 1.05f;
-            const float4 s = sample_atlas<SC, COUNT>(S.ad, S.chunks, S.culled, S.objects, objInvBase + S.objectStart * 16,
-                                                     S.tiles, static_cast<const SC*>(S.color), S.atlasDepth, hp, n,
-                                                     thr, c);
-            const float dist = fmaxf(hitTime + S.g.cascadeVoxelSize[hitCascade] * 0.5f, 0.0f);
-            Texel<SR>::st4(outRad, e, make_float4(s.x, s.y, s.z, 0.f));
-            Texel<SR>::st4(outDD, e, make_float4(dir.x, dir.y, dir.z, dist));
-            if (flags) flags[e] = 1;
-        }
-    } else {
-        store_nonhit<SR>(A, S, skyFaces, outRad, outDD, flags, e, dir, false);
-    }
-}
+// A front hit as the wave's groups read it: hit point, normal, weight threshold, object list
+struct HitLds {
+    float hp[3][64], n[3][64], thr[64];
+    uint32_t list[64], count[64];
+};
 
-// One ray per lane: the sorted front hits (`order`, grouped by atlas chunk, so the object and tile
-// loops of a wave run in step), or every ray (MODE 0: 64 rays of a probe per wave; MODE 1 and 2:
-// the flat ray list of a batch, as in march_kernel).
+// Radiance of the front hits (SDFCommon.glsl:172-184, GISDFRays.comp:89-119). A wave takes the 64 rays the
+// march's wave traced. First one ray per lane: the hit point, the normal and the chunk's object list.
+// Then eight lanes per hit, eight hits at a time: the lanes test eight objects of the list at once, and
+// for each object that holds the point take one tile each, so the chain of dependent loads per hit is
+// that of one object and one tile, and a wave waits for the longest of 8 lists instead of 64.
+// One lane per hit, with the hits counting-sorted by chunk so that a wave's lists agree, took
+// 479 us for the 2.4 M hits of a 32x16x32x256 volume and 300 us more for the sort: its keys, a
+// histogram with an atomic per chunk of each wave, a scan, a scatter, and records and outputs at
+// scattered addresses; the whole trace 1,652 us against 1,513 now (shade 487), 102 against 68 for a
+// 13x7x11x100 volume in FP16 and 120 against 90 for an 8x8x8x64 one. Bound at the large size: L2
+// misses (19.6 M lines in 487 us, 5.1 TB/s), a third of them the normals'.
 template <class SS, class SC, class SR, bool COUNT, int MODE>
 __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __restrict__ objInvBase,
-                                                    const float4* __restrict__ recA, const float2* __restrict__ recB,
-                                                    const uint32_t* __restrict__ order,
-                                                    const uint32_t* __restrict__ hitCount,
+                                                    const float4* __restrict__ recA, const uint8_t* __restrict__ recC,
                                                     unsigned long long* __restrict__ counters) {
+    __shared__ HitLds lds[4];
+    HitLds& L = lds[threadIdx.x >> 6];
+    const int lane = threadIdx.x & 63;
     const long long gid = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     Counts c = {0, 0, 0, 0, 0, 0, 0};
-    bool active;
-    if (MODE == 2) {  // ray order only: a wave lies in one volume
-        active = gid < A.totalRays;
-        const LuxgiTraceVolume& v = A.vols[batch_volume<2>(A, gid)];
-        const int R = v.uniform.raysPerProbe;
-        const long long local = gid - v.rayStart;
-        active = active && local >= 0 && local < volume_rays(v);
-        if (active)
-            shade_ray<SS, SC, SR, COUNT>(A, A.scenes[v.scene], v, int(local / R), int(local % R), (size_t)gid,
-                                         objInvBase, recA, recB, c);
-    } else if (MODE == 1 || order) {  // a flat ray id
-        long long rid = -1;
-        if (order) {
-            if (gid < (long long)*hitCount) rid = order[gid];
-        } else if (gid < A.totalRays) {
-            rid = gid;
+    const LuxgiTraceVolume* v;
+    int probe, ray;
+    size_t rid;
+    const bool valid = find_ray<MODE>(A, gid, v, probe, ray, rid);
+    const TraceScene& S = MODE == 2 ? A.scenes[v->scene] : A.scene;
+    float4 ra = make_float4(-1.f, 0.f, 0.f, 0.f);
+    if (valid) ra = recA[rid];
+    const bool hit = ra.x >= 0.0f;
+    uint32_t list = 0, count = 0;
+    f3 hp = mk(0.f, 0.f, 0.f), n = hp;
+    float thr = 0.0f;
+    if (hit) {
+        f3 origin, dir;
+        ray_setup(A, *v, probe, ray, origin, dir);
+        hp = origin + dir * ra.x;
+        list = S.chunks[atlas_chunk(S.ad, hp)];
+        if (list != 0) {
+            count = S.culled[list];
+            if (count > S.ad.objectsCount) count = 0;
+            ++list;
         }
-        active = rid >= 0;
-        if (active) {
-            if constexpr (MODE == 1) {
-                const LuxgiTraceVolume& v = A.vols[trace_volume_of(A.vols, A.nVols, rid)];
-                const int R = v.uniform.raysPerProbe;
-                const long long local = rid - v.rayStart;
-                active = local >= 0 && local < volume_rays(v);
-                if (active)
-                    shade_ray<SS, SC, SR, COUNT>(A, A.scene, v, int(local / R), int(local % R), (size_t)rid,
-                                                 objInvBase, recA, recB, c);
-            } else {
-                shade_ray<SS, SC, SR, COUNT>(A, A.scene, A.vol, int(rid / A.R), int(rid % A.R), (size_t)rid,
-                                             objInvBase, recA, recB, c);
-            }
+        thr = S.g.cascadeVoxelSize[recC[rid]] * 1.05f;
+        const SS* sdf = static_cast<const SS*>(S.sdf);
+        const int texW = S.res * (int)S.g.cascadesCount;
+        const float o = 1.0f / S.g.resolution;
+        const float tx = ra.y, uy = ra.z, uz = ra.w;
+        auto nl = [&](float u_, float v_, float w_) {
+            if (S.refine) return refine_lookup(A, S, texW, S.res, S.res, u_, v_, w_);
+            if (A.fineLayout == LUXGI_LAYOUT_BRICK4)
+                return sample3d_brick4<SS>(sdf, texW, S.res, S.res, u_, v_, w_, S.brickScale);
+            if (A.fineLayout == LUXGI_LAYOUT_CELL8) return sample3d_cell8<SS>(sdf, texW, S.res, S.res, u_, v_, w_);
+            return sample_volume<SS>(sdf, texW, S.res, S.res, u_, v_, w_);
+        };
+        const float xp = nl(tx + o, uy, uz), xn = nl(tx - o, uy, uz);
+        const float yp = nl(tx, uy + o, uz), yn = nl(tx, uy - o, uz);
+        const float zp = nl(tx, uy, uz + o), zn = nl(tx, uy, uz - o);
+        n = normalize3(mk(xp - xn, yp - yn, zp - zn));
+        if (COUNT) c.normals++;
+    }
+    // the hits with a list, packed
+    const unsigned long long todo = __ballot(count > 0);
+    const int total = __popcll(todo), rank = __popcll(todo & ((1ull << lane) - 1ull));
+    if (count > 0) {
+        L.hp[0][rank] = hp.x; L.hp[1][rank] = hp.y; L.hp[2][rank] = hp.z;
+        L.n[0][rank] = n.x; L.n[1][rank] = n.y; L.n[2][rank] = n.z;
+        L.thr[rank] = thr;
+        L.list[rank] = list;
+        L.count[rank] = count;
+    }
+    wave_lds_fence();
+    const int t = lane & 7;
+    for (int k0 = 0; k0 < total; k0 += 8) {
+        const int k = k0 + (lane >> 3);
+        f3 p = mk(0.f, 0.f, 0.f), pn = p;
+        float pt = 0.0f;
+        uint32_t pl = 0, pc = 0;
+        if (k < total) {
+            p = mk(L.hp[0][k], L.hp[1][k], L.hp[2][k]);
+            pn = mk(L.n[0][k], L.n[1][k], L.n[2][k]);
+            pt = L.thr[k];
+            pl = L.list[k];
+            pc = L.count[k];
         }
-    } else {
-        const int Rp = (A.R + 63) & ~63;
-        const int probe = int(gid / Rp), ray = int(gid % Rp);
-        active = probe < A.P && ray < A.R;
-        if (active)
-            shade_ray<SS, SC, SR, COUNT>(A, A.scene, A.vol, probe, ray, (size_t)probe * A.R + ray, objInvBase, recA,
-                                         recB, c);
+        const float4 s = sample_atlas_group<SC, COUNT>(S.ad, S.culled, S.objects, objInvBase + S.objectStart * 16,
+                                                       S.tiles, static_cast<const SC*>(S.color), S.atlasDepth, p, pn,
+                                                       pt, pl, pc, c);
+        if (k < total && t == 0) {  // the slot's hit is read: its result takes its place
+            L.hp[0][k] = s.x;
+            L.hp[1][k] = s.y;
+            L.hp[2][k] = s.z;
+        }
+    }
+    wave_lds_fence();
+    if (hit) {
+        float4 rad = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (count > 0) rad = make_float4(L.hp[0][rank], L.hp[1][rank], L.hp[2][rank], 0.f);
+        Texel<SR>::st4(static_cast<SR*>(v->rays.radiance), (size_t)probe * v->rays.width + ray, rad);
     }
     if (COUNT) {
-        __shared__ unsigned long long sc[8];
-        if (threadIdx.x < 8) sc[threadIdx.x] = 0;
+        __shared__ unsigned long long sc[4];
+        if (threadIdx.x < 4) sc[threadIdx.x] = 0;
         __syncthreads();
-        if (active) {
-            atomicAdd(&sc[2], c.normals);
-            atomicAdd(&sc[3], c.objects);
-            atomicAdd(&sc[4], c.tiles);
-            atomicAdd(&sc[5], 1ull);
-            atomicAdd(&sc[7], c.hits);
-        }
+        atomicAdd(&sc[0], c.normals);
+        atomicAdd(&sc[1], c.objects);
+        atomicAdd(&sc[2], c.tiles);
+        atomicAdd(&sc[3], valid ? 1ull : 0ull);
         __syncthreads();
-        if (threadIdx.x < 8 && threadIdx.x != 0 && threadIdx.x != 1 && threadIdx.x != 6)
-            atomicAdd(&counters[threadIdx.x], sc[threadIdx.x]);
-    }
-}
-
-// counting sort of the rays by hit chunk: zero the bins, exclusive scan, scatter
-__global__ void zero_bins_kernel(uint32_t* __restrict__ bins, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) bins[i] = 0u;
-}
-
-constexpr int kScanBlock = 1024;
-constexpr int kScanBlocks = (kChunkBins + kScanBlock - 1) / kScanBlock;
-static_assert(kScanBlocks <= 64, "the block totals are scanned by one wave");
-
-// order[start of the chunk + slot] = ray for every front hit; block 0 also stores the hit count
-__global__ __launch_bounds__(256) void scatter_hits_kernel(const uint2* __restrict__ keys,
-                                                           const uint32_t* __restrict__ starts,
-                                                           const uint32_t* __restrict__ totals,
-                                                           uint32_t* __restrict__ hitCount,
-                                                           uint32_t* __restrict__ order, long long n) {
-    __shared__ uint32_t blockStart[64];
-    if (threadIdx.x < 64) {
-        const uint32_t t = threadIdx.x < kScanBlocks ? totals[threadIdx.x] : 0u;
-        const uint32_t x = wave_inclusive_scan(t);
-        blockStart[threadIdx.x] = x - t;
-        if (blockIdx.x == 0 && threadIdx.x == 63) *hitCount = x;
-    }
-    __syncthreads();
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const uint2 k = keys[i];
-        if (k.x != kNoChunk) order[blockStart[k.x / kScanBlock] + starts[k.x] + k.y] = (uint32_t)i;
+        if (threadIdx.x < 4) atomicAdd(&counters[2 + threadIdx.x], sc[threadIdx.x]);
     }
 }
 
@@ -594,13 +524,9 @@ using namespace luxgi;
 static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 struct TraceWorkspace {
-    float* inv;
-    float4* recA;
-    float2* recB;
-    uint2* keys;      // hit sort: (chunk, slot in the chunk) per ray
-    uint32_t* bins;   // per-chunk hit counts, then their in-block exclusive scan
-    uint32_t* totals; // scan block totals, then the hit count at [kScanBlocks]
-    uint32_t* order;  // front hits in chunk order
+    float* inv;     // per-object inverse transforms
+    float4* recA;   // per-ray hit records
+    uint8_t* recC;  // and their cascades
 };
 
 static size_t trace_workspace_layout(size_t rays, int64_t objects, char* base, TraceWorkspace* w) {
@@ -609,16 +535,8 @@ static size_t trace_workspace_layout(size_t rays, int64_t objects, char* base, T
     off += align256((size_t)(objects > 0 ? objects : 0) * 16 * sizeof(float));
     if (w) w->recA = reinterpret_cast<float4*>(base + off);
     off += align256(rays * sizeof(float4));
-    if (w) w->recB = reinterpret_cast<float2*>(base + off);
-    off += align256(rays * sizeof(float2));
-    if (w) w->keys = reinterpret_cast<uint2*>(base + off);
-    off += align256(rays * sizeof(uint2));
-    if (w) w->bins = reinterpret_cast<uint32_t*>(base + off);
-    off += align256((size_t)kChunkBins * sizeof(uint32_t));
-    if (w) w->totals = reinterpret_cast<uint32_t*>(base + off);
-    off += align256((size_t)(kScanBlocks + 1) * sizeof(uint32_t));
-    if (w) w->order = reinterpret_cast<uint32_t*>(base + off);
-    off += align256(rays * sizeof(uint32_t));
+    if (w) w->recC = reinterpret_cast<uint8_t*>(base + off);
+    off += align256(rays);
     return off;
 }
 
@@ -629,14 +547,12 @@ extern "C" size_t luxgi_ddgi_trace_workspace_size(const LuxgiDDGIUniform* u, int
     return trace_workspace_layout(P * R, objectCapacity, nullptr, nullptr);
 }
 
-// The kernels of one trace: object inverses, (hit-sort bins), march, (scan + scatter), shade. MODE 0:
-// one volume, 1: a batch over A.scene, 2: a batch over per-volume scenes (A.scenes, nScenes of them,
-// at most maxObjects objects each).
+// The kernels of one trace: object inverses, march, shade. MODE 0: one volume, 1: a batch over A.scene,
+// 2: a batch over per-volume scenes (A.scenes, nScenes of them, at most maxObjects objects each).
 template <class SS, class SC, class SR, bool COUNT, int MODE>
 static int launch_trace(const TraceArgs& A, int nScenes, int maxObjects, const TraceWorkspace& w,
                         unsigned long long* counters, hipStream_t st) {
-    const long long nRays = MODE != 0 ? A.totalRays : (long long)A.P * A.R;
-    const long long lanes = MODE != 0 ? nRays : (long long)A.P * ((A.R + 63) & ~63);
+    const long long lanes = MODE != 0 ? A.totalRays : (long long)A.P * ((A.R + 63) & ~63);
     if (MODE == 2) {
         if (maxObjects > 0) {
             hipLaunchKernelGGL(trace_prepare_scenes_kernel, dim3((maxObjects + 255) / 256, nScenes), dim3(256), 0, st,
@@ -648,33 +564,19 @@ static int launch_trace(const TraceArgs& A, int nScenes, int maxObjects, const T
                            st, A.scene.objects, A.scene.objectCapacity, w.inv);
         LUXGI_LAUNCH_CHECK();
     }
-    if (A.sortHits) {
-        hipLaunchKernelGGL(zero_bins_kernel, dim3((kChunkBins + 255) / 256), dim3(256), 0, st, w.bins, kChunkBins);
-        LUXGI_LAUNCH_CHECK();
-    }
-    const dim3 mgrid((int)((lanes + 255) / 256));
+    const dim3 grid((int)((lanes + 255) / 256));
     if (A.fineLayout == LUXGI_LAYOUT_BRICK4)
-        hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_BRICK4, MODE>), mgrid, dim3(256), 0, st, A, w.recA,
-                           w.recB, w.keys, w.bins, counters);
+        hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_BRICK4, MODE>), grid, dim3(256), 0, st, A, w.recA,
+                           w.recC, counters);
     else if (A.fineLayout == LUXGI_LAYOUT_CELL8)
-        hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_CELL8, MODE>), mgrid, dim3(256), 0, st, A, w.recA,
-                           w.recB, w.keys, w.bins, counters);
+        hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_CELL8, MODE>), grid, dim3(256), 0, st, A, w.recA,
+                           w.recC, counters);
     else
-        hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_LINEAR, MODE>), mgrid, dim3(256), 0, st, A, w.recA,
-                           w.recB, w.keys, w.bins, counters);
+        hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_LINEAR, MODE>), grid, dim3(256), 0, st, A, w.recA,
+                           w.recC, counters);
     LUXGI_LAUNCH_CHECK();
-    if (A.sortHits) {
-        hipLaunchKernelGGL(block_scan_kernel<kScanBlock>, dim3(kScanBlocks), dim3(kScanBlock), 0, st, w.bins, w.bins,
-                           w.totals, kChunkBins);
-        LUXGI_LAUNCH_CHECK();
-        hipLaunchKernelGGL(scatter_hits_kernel, dim3((int)((nRays + 255) / 256)), dim3(256), 0, st, w.keys, w.bins,
-                           w.totals, w.totals + kScanBlocks, w.order, nRays);
-        LUXGI_LAUNCH_CHECK();
-    }
-    // sorted: one lane per ray covers every possible hit count; the lanes past the count exit
-    const long long shadeLanes = A.sortHits ? nRays : lanes;
-    hipLaunchKernelGGL((shade_kernel<SS, SC, SR, COUNT, MODE>), dim3((int)((shadeLanes + 255) / 256)), dim3(256), 0, st,
-                       A, w.inv, w.recA, w.recB, A.sortHits ? w.order : nullptr, w.totals + kScanBlocks, counters);
+    hipLaunchKernelGGL((shade_kernel<SS, SC, SR, COUNT, MODE>), grid, dim3(256), 0, st, A, w.inv, w.recA, w.recC,
+                       counters);
     LUXGI_LAUNCH_CHECK();
     return LUXGI_OK;
 }
@@ -746,7 +648,6 @@ static int trace_scene_args(const LuxgiGlobalSDFData* g, const LuxgiSDFVolume* v
     A.hitEps = p->hitEpsilon;
     A.fineLayout = vol->layout;
     if (p->shadeOrder != 0 && p->shadeOrder != 1) return LUXGI_ERR_INVALID_ARGUMENT;
-    A.sortHits = !count && p->shadeOrder == 0;  // the counting run shades in ray order
     A.vols = nullptr;
     A.nVols = 0;
     A.totalRays = 0;
@@ -937,7 +838,6 @@ extern "C" int luxgi_ddgi_trace_sdf_scenes(const LuxgiTraceSceneBatch* batch, co
     A.maxSteps = p->maxSteps > 0 ? p->maxSteps : 250;
     A.hitEps = p->hitEpsilon;
     A.fineLayout = batch->sdfLayout;
-    A.sortHits = 0;  // shaded in ray order: a wave stays within one volume and scene
     A.vols = volumes;
     A.nVols = batch->volumeCount;
     A.totalRays = batch->totalRays;

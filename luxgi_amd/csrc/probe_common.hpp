@@ -10,13 +10,8 @@ namespace luxgi {
 
 constexpr float kPiF = 3.1415926535897932384626433832795f;  // Common/Math.glsl:7
 
-// GLSL normalize / pow as the hardware evaluates them: reciprocal square root (v_rsq_f32) and
-// 2^(y log2 x) (v_log_f32, v_exp_f32), each within a few ulp of the correctly rounded value --
-// inside the precision GLSL grants these built-ins.
-__device__ __forceinline__ f3 fast_normalize(f3 a) {
-    const float r = __builtin_amdgcn_rsqf(dot3(a, a));
-    return mk(a.x * r, a.y * r, a.z * r);
-}
+// GLSL pow as the hardware evaluates it, 2^(y log2 x) (v_log_f32, v_exp_f32): within a few ulp of the
+// correctly rounded value -- inside the precision GLSL grants the built-in.
 __device__ __forceinline__ float fast_pow(float x, float y) {  // x >= 0
     return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x));
 }
@@ -51,13 +46,6 @@ __device__ __forceinline__ float2 atlas_coord(f3 dir, int2 tile, const AtlasGeom
 }
 __host__ __device__ inline AtlasGeom atlas_geom(int width, int height, int side) {
     return AtlasGeom{width, height, side, (width - 2) / (side + 2), 1.0f / float(width), 1.0f / float(height)};
-}
-
-// i modulo n; the division only where i is outside [0, n)
-__device__ __forceinline__ int wrap_index(int i, int n) {
-    if ((unsigned)i < (unsigned)n) return i;
-    const int m = i % n;
-    return m < 0 ? m + n : m;
 }
 
 // A row of two neighbouring texels, the left one at i.

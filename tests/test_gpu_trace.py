@@ -86,6 +86,27 @@ def test_trace_matches_oracle_config1(max_steps, hit_eps):
     assert (fl == 1).mean() > 0.3 and (fl == 0).mean() > 0.01  # the scene has hits and misses
 
 
+@pytest.mark.parametrize("rays", [1, 7, 63, 65])
+def test_trace_shade_groups_at_wave_and_list_edges(rays):
+    """Waves with 1, 7, 63 and 64 + 1 rays (hits in partly filled groups of eight lanes) over a scene whose
+    chunks hold 1 to 16 objects (lists of 8, 9 and 16, the groups' steps). Tolerances as in the other
+    trace tests."""
+    prims = scene.scene_random(n=60, seed=9, size_range=(0.4, 1.0))
+    sdf = scene.bake_sdf_numpy(prims, 64)
+    g = abi.make_sdf_data(resolution=64)
+    mip = oracle.sdf_mip(sdf, 64, max_distance=2.0, flood_passes=4)
+    atlas = scene.build_atlas(prims, resolution=512, tile=16, seed=3, threshold=1.05 * 2.0 / 64)
+    lists = set(atlas.culled[atlas.chunks[atlas.chunks > 0]].tolist())
+    assert {1, 7, 8, 9, 16} <= lists
+    u = _scenes.small_uniform(rays=rays, counts=(9, 8, 7))
+    p = _scenes.trace_params(rot_seed=17)
+    gpu = _gpu_trace(u, g, sdf, mip, atlas, p)
+    ref = _scenes.oracle_trace(u, g, sdf, mip, atlas, p)
+    _compare(u, g, gpu, ref, 2.0 / 64)
+    lit = (gpu[2] == 1) & (np.abs(gpu[0][..., :3]).sum(-1) > 0)
+    assert lit.mean() > 0.1
+
+
 def test_trace_unorm8_atlas_and_offsets():
     prims, sdf, mip, g, atlas = _scenes.small_scene(color_storage=abi.STORAGE_UNORM8)
     u = _scenes.small_uniform(rays=96, counts=(5, 4, 6))

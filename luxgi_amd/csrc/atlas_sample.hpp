@@ -221,50 +221,73 @@ __device__ __forceinline__ float4 sample_atlas_group(const LuxgiSurfaceAtlasData
     return make_float4(res.x * a, res.y * a, res.z * a, res.w);
 }
 
-// sampleGlobalSurfaceAtlas (AtlasCommon.glsl:115-157), debug = false: (rgb / max(a, 1e-4), a) with a
-// the summed tile weights, (0, 0, 0, 0) when the chunk has no list
+// object list of a world position's chunk (AtlasCommon.glsl:124-131): the first id's place in `culled`;
+// count 0 without a list
+__device__ __forceinline__ void atlas_list(const LuxgiSurfaceAtlasData& ad, const uint32_t* __restrict__ chunks,
+                                           const uint32_t* __restrict__ culled, f3 wp, uint32_t& list, uint32_t& count) {
+    list = chunks[atlas_chunk(ad, wp)];
+    count = 0;
+    if (list != 0) {
+        count = culled[list];
+        if (count > ad.objectsCount) count = 0;
+        ++list;
+    }
+}
+
+// The lookups of a wave's lanes as its groups of eight read them: point, normal, weight threshold, list
+struct AtlasQueryLds {
+    float p[3][64], n[3][64], thr[64];
+    uint32_t list[64], count[64];
+};
+
+// The surface-atlas lookup of every lane with count > 0 (see atlas_list; (0, 0, 0, 0) for the others):
+// (rgb / max(a, 1e-4), a) with a the summed tile weights (AtlasCommon.glsl:115-157, debug = false).
+// The whole wave calls it; its lookups are packed and worked off eight at a time, eight lanes each,
+// so the chain of dependent loads per lookup is that of one object and one tile and the wave waits
+// for the longest of eight lists at a time instead of 64.
 template <class SC, bool COUNT>
-__device__ float4 sample_atlas(const LuxgiSurfaceAtlasData& ad, const uint32_t* __restrict__ chunks,
-                               const uint32_t* __restrict__ culled, const LuxgiAtlasObject* __restrict__ objects,
-                               const float* __restrict__ objInv, const LuxgiAtlasTile* __restrict__ tiles,
-                               const SC* __restrict__ color, const float* __restrict__ depth, f3 wp, f3 wn,
-                               float threshold, Counts& c) {
-    float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint32_t start = chunks[atlas_chunk(ad, wp)];
-    if (start == 0) return make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t count = culled[start];
-    if (count > ad.objectsCount) return make_float4(0.f, 0.f, 0.f, 0.f);
-    start++;
-    for (uint32_t oi = 0; oi < count; ++oi) {
-        const uint32_t id = culled[start++];
-        const LuxgiAtlasObject* o = objects + id;
-        if (COUNT) c.objects++;
-        const float4 bs = *reinterpret_cast<const float4*>(o->objectBounds);
-        if (len3(mk(bs.x, bs.y, bs.z) - wp) > bs.w) continue;
-        const float* inv = objInv + (size_t)id * 16;
-        float m[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) m[k] = inv[k];
-        const float4 l4 = mat4_mul4(m, make_float4(wp.x, wp.y, wp.z, 1.0f));
-        const f3 lp = mk(l4.x, l4.y, l4.z);
-        const float4 e = *reinterpret_cast<const float4*>(o->extends);
-        if (fabsf(lp.x) > e.x + threshold || fabsf(lp.y) > e.y + threshold || fabsf(lp.z) > e.z + threshold) continue;
-        f3 ln = mk(m[0] * wn.x + m[4] * wn.y + m[8] * wn.z, m[1] * wn.x + m[5] * wn.y + m[9] * wn.z,
-                   m[2] * wn.x + m[6] * wn.y + m[10] * wn.z);
-        ln = fast_normalize(ln);
-        for (int t = 0; t < 6; ++t) {
-            const uint32_t to = o->tileOffset[t];
-            if (to != 0) {
-                float4 s = sample_tile<SC, COUNT>(ad, tiles + to, color, depth, lp, ln, threshold, c);
-                res.x += s.x;
-                res.y += s.y;
-                res.z += s.z;
-                res.w += s.w;
-            }
+__device__ __forceinline__ float4 sample_atlas_wave(const LuxgiSurfaceAtlasData& ad, const uint32_t* __restrict__ culled,
+                                                    const LuxgiAtlasObject* __restrict__ objects,
+                                                    const float* __restrict__ objInv,
+                                                    const LuxgiAtlasTile* __restrict__ tiles,
+                                                    const SC* __restrict__ color, const float* __restrict__ depth,
+                                                    AtlasQueryLds& L, f3 wp, f3 wn, float threshold, uint32_t list,
+                                                    uint32_t count, Counts& c) {
+    const int lane = threadIdx.x & 63;
+    const unsigned long long todo = __ballot(count > 0);
+    const int total = __popcll(todo), rank = __popcll(todo & ((1ull << lane) - 1ull));
+    if (count > 0) {
+        L.p[0][rank] = wp.x; L.p[1][rank] = wp.y; L.p[2][rank] = wp.z;
+        L.n[0][rank] = wn.x; L.n[1][rank] = wn.y; L.n[2][rank] = wn.z;
+        L.thr[rank] = threshold;
+        L.list[rank] = list;
+        L.count[rank] = count;
+    }
+    wave_lds_fence();
+    for (int k0 = 0; k0 < total; k0 += 8) {
+        const int k = k0 + (lane >> 3);
+        f3 p = mk(0.f, 0.f, 0.f), n = p;
+        float pt = 0.0f;
+        uint32_t pl = 0, pc = 0;
+        if (k < total) {
+            p = mk(L.p[0][k], L.p[1][k], L.p[2][k]);
+            n = mk(L.n[0][k], L.n[1][k], L.n[2][k]);
+            pt = L.thr[k];
+            pl = L.list[k];
+            pc = L.count[k];
+        }
+        const float4 s = sample_atlas_group<SC, COUNT>(ad, culled, objects, objInv, tiles, color, depth, p, n, pt, pl,
+                                                       pc, c);
+        if (k < total && (lane & 7) == 0) {  // the slot's lookup is read: its result takes its place
+            L.p[0][k] = s.x;
+            L.p[1][k] = s.y;
+            L.p[2][k] = s.z;
+            L.thr[k] = s.w;
         }
     }
-    const float a = fmaxf(res.w, 0.0001f);
-    return make_float4(res.x / a, res.y / a, res.z / a, res.w);
+    wave_lds_fence();
+    if (count == 0) return make_float4(0.f, 0.f, 0.f, 0.f);
+    return make_float4(L.p[0][rank], L.p[1][rank], L.p[2][rank], L.thr[rank]);
 }
 
 // cubemap lookup (RGBA32F faces +X -X +Y -Y +Z -Z), bilinear inside the face, clamp-to-edge

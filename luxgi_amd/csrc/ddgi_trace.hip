@@ -389,17 +389,9 @@ __global__ __launch_bounds__(256) void march_kernel(TraceArgs A, float4* __restr
     }
 }
 
-// A front hit as the wave's groups read it: hit point, normal, weight threshold, object list
-struct HitLds {
-    float hp[3][64], n[3][64], thr[64];
-    uint32_t list[64], count[64];
-};
-
 // Radiance of the front hits (SDFCommon.glsl:172-184, GISDFRays.comp:89-119). A wave takes the 64 rays the
-// march's wave traced. First one ray per lane: the hit point, the normal and the chunk's object list.
-// Then eight lanes per hit, eight hits at a time: the lanes test eight objects of the list at once, and
-// for each object that holds the point take one tile each, so the chain of dependent loads per hit is
-// that of one object and one tile, and a wave waits for the longest of 8 lists instead of 64.
+// march's wave traced: first one ray per lane, the hit point, the normal and the chunk's object list,
+// then eight lanes per hit, eight hits at a time (sample_atlas_wave).
 // One lane per hit, with the hits counting-sorted by chunk so that a wave's lists agree, took
 // 479 us for the 2.4 M hits of a 32x16x32x256 volume and 300 us more for the sort: its keys, a
 // histogram with an atomic per chunk of each wave, a scan, a scatter, and records and outputs at
@@ -410,9 +402,7 @@ template <class SS, class SC, class SR, bool COUNT, int MODE>
 __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __restrict__ objInvBase,
                                                     const float4* __restrict__ recA, const uint8_t* __restrict__ recC,
                                                     unsigned long long* __restrict__ counters) {
-    __shared__ HitLds lds[4];
-    HitLds& L = lds[threadIdx.x >> 6];
-    const int lane = threadIdx.x & 63;
+    __shared__ AtlasQueryLds lds[4];
     const long long gid = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     Counts c = {0, 0, 0, 0, 0, 0, 0};
     const LuxgiTraceVolume* v;
@@ -430,12 +420,7 @@ __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __
         f3 origin, dir;
         ray_setup(A, *v, probe, ray, origin, dir);
         hp = origin + dir * ra.x;
-        list = S.chunks[atlas_chunk(S.ad, hp)];
-        if (list != 0) {
-            count = S.culled[list];
-            if (count > S.ad.objectsCount) count = 0;
-            ++list;
-        }
+        atlas_list(S.ad, S.chunks, S.culled, hp, list, count);
         thr = S.g.cascadeVoxelSize[recC[rid]] * 1.05f;
         const SS* sdf = static_cast<const SS*>(S.sdf);
         const int texW = S.res * (int)S.g.cascadesCount;
@@ -454,45 +439,12 @@ __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __
         n = normalize3(mk(xp - xn, yp - yn, zp - zn));
         if (COUNT) c.normals++;
     }
-    // the hits with a list, packed
-    const unsigned long long todo = __ballot(count > 0);
-    const int total = __popcll(todo), rank = __popcll(todo & ((1ull << lane) - 1ull));
-    if (count > 0) {
-        L.hp[0][rank] = hp.x; L.hp[1][rank] = hp.y; L.hp[2][rank] = hp.z;
-        L.n[0][rank] = n.x; L.n[1][rank] = n.y; L.n[2][rank] = n.z;
-        L.thr[rank] = thr;
-        L.list[rank] = list;
-        L.count[rank] = count;
-    }
-    wave_lds_fence();
-    const int t = lane & 7;
-    for (int k0 = 0; k0 < total; k0 += 8) {
-        const int k = k0 + (lane >> 3);
-        f3 p = mk(0.f, 0.f, 0.f), pn = p;
-        float pt = 0.0f;
-        uint32_t pl = 0, pc = 0;
-        if (k < total) {
-            p = mk(L.hp[0][k], L.hp[1][k], L.hp[2][k]);
-            pn = mk(L.n[0][k], L.n[1][k], L.n[2][k]);
-            pt = L.thr[k];
-            pl = L.list[k];
-            pc = L.count[k];
-        }
-        const float4 s = sample_atlas_group<SC, COUNT>(S.ad, S.culled, S.objects, objInvBase + S.objectStart * 16,
-                                                       S.tiles, static_cast<const SC*>(S.color), S.atlasDepth, p, pn,
-                                                       pt, pl, pc, c);
-        if (k < total && t == 0) {  // the slot's hit is read: its result takes its place
-            L.hp[0][k] = s.x;
-            L.hp[1][k] = s.y;
-            L.hp[2][k] = s.z;
-        }
-    }
-    wave_lds_fence();
-    if (hit) {
-        float4 rad = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (count > 0) rad = make_float4(L.hp[0][rank], L.hp[1][rank], L.hp[2][rank], 0.f);
-        Texel<SR>::st4(static_cast<SR*>(v->rays.radiance), (size_t)probe * v->rays.width + ray, rad);
-    }
+    const float4 s = sample_atlas_wave<SC, COUNT>(S.ad, S.culled, S.objects, objInvBase + S.objectStart * 16, S.tiles,
+                                                  static_cast<const SC*>(S.color), S.atlasDepth, lds[threadIdx.x >> 6],
+                                                  hp, n, thr, list, count, c);
+    if (hit)
+        Texel<SR>::st4(static_cast<SR*>(v->rays.radiance), (size_t)probe * v->rays.width + ray,
+                       make_float4(s.x, s.y, s.z, 0.f));
     if (COUNT) {
         __shared__ unsigned long long sc[4];
         if (threadIdx.x < 4) sc[threadIdx.x] = 0;

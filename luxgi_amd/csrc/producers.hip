@@ -160,48 +160,60 @@ __global__ __launch_bounds__(256) void reflection_kernel(ReflArgsP A, const floa
                                                          const float* __restrict__ skyFaces,
                                                          const SA* __restrict__ irr, const SA* __restrict__ dep,
                                                          void* __restrict__ out) {
+    __shared__ AtlasQueryLds lds[4];
     const int x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (x >= A.W || y >= A.H) return;
     const size_t e = (size_t)y * A.W + x;
-    const float d = depth[e];
-    if (d == 1.0f) return;  // sky: the reference leaves the texel as it was
-    const float tu = (float(x) + 0.5f) / float(A.W), tv = (float(y) + 0.5f) / float(A.H);
-    f3 wp = world_from_depth(tu, tv, d, A.p.viewProjInv);
-    const float roughness = pbr[e * 4 + 1];
-    const float2 on = reinterpret_cast<const float2*>(normals)[2 * e];
-    const f3 n = oct_decode(on.x, on.y);
-    const f3 Wo = normalize3(mk(A.p.cameraPosition[0], A.p.cameraPosition[1], A.p.cameraPosition[2]) - wp);
-    wp = wp + n * A.g.cascadeVoxelSize[0];  // self-occlusion bias
+    const float d = x < A.W && y < A.H ? depth[e] : 1.0f;
+    const bool on = d != 1.0f;  // sky: the reference leaves the texel as it was
     float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
-    bool traceRay = true;
-    f3 R;
-    if (roughness < 0.05f) {  // MIRROR_REFLECTIONS_ROUGHNESS_THRESHOLD
-        R = reflect3(mk(-Wo.x, -Wo.y, -Wo.z), n);
-    } else if (roughness > 0.45f && A.p.approximateWithDDGI == 1u) {  // DDGI_REFLECTIONS_ROUGHNESS_THRESHOLD
-        R = reflect3(mk(-Wo.x, -Wo.y, -Wo.z), n);
-        traceRay = false;
-        if (A.ddgi) {
-            const f3 ir = sample_irradiance<SA>(A.u, A.irrG, A.depG, wp, R, Wo, irr, dep, A.rl);
-            col = make_float4(A.p.roughDDGIIntensity * ir.x, A.p.roughDDGIIntensity * ir.y,
-                              A.p.roughDDGIIntensity * ir.z, 0.0f);
-        }
-    } else {
-        const float ex = blue_noise(sobol, scr, x, y, int(A.p.numFrames), 0) * A.p.trim;
-        const float ey = blue_noise(sobol, scr, x, y, int(A.p.numFrames), 1) * A.p.trim;
-        const f3 Hh = importance_sample_ggx(ex, ey, n, roughness);
-        R = reflect3(mk(-Wo.x, -Wo.y, -Wo.z), Hh);
-    }
-    if (traceRay) {
-        const SdfHitTime h = trace_global_sdf<SS, FL>(sdf, A.g, wp, R, kGlobalSdfWorldSize, 0.0f, A.maxSteps);
-        if (h.time >= 0.0f) {
-            Counts c{};
-            const f3 hp = wp + R * h.time;
-            col = sample_atlas<SC, false>(A.ad, chunks, culled, objects, objInv, tiles, color, atlasDepth, hp,
-                                           mk(-R.x, -R.y, -R.z), A.g.cascadeVoxelSize[h.cascade] * 1.05f, c);
+    f3 hp = mk(0.f, 0.f, 0.f), R = hp;
+    float thr = 0.0f;
+    uint32_t list = 0, count = 0;
+    bool hit = false;
+    if (on) {
+        const float tu = (float(x) + 0.5f) / float(A.W), tv = (float(y) + 0.5f) / float(A.H);
+        f3 wp = world_from_depth(tu, tv, d, A.p.viewProjInv);
+        const float roughness = pbr[e * 4 + 1];
+        const float2 oct = reinterpret_cast<const float2*>(normals)[2 * e];
+        const f3 n = oct_decode(oct.x, oct.y);
+        const f3 Wo = normalize3(mk(A.p.cameraPosition[0], A.p.cameraPosition[1], A.p.cameraPosition[2]) - wp);
+        wp = wp + n * A.g.cascadeVoxelSize[0];  // self-occlusion bias
+        bool traceRay = true;
+        if (roughness < 0.05f) {  // MIRROR_REFLECTIONS_ROUGHNESS_THRESHOLD
+            R = reflect3(mk(-Wo.x, -Wo.y, -Wo.z), n);
+        } else if (roughness > 0.45f && A.p.approximateWithDDGI == 1u) {  // DDGI_REFLECTIONS_ROUGHNESS_THRESHOLD
+            R = reflect3(mk(-Wo.x, -Wo.y, -Wo.z), n);
+            traceRay = false;
+            if (A.ddgi) {
+                const f3 ir = sample_irradiance<SA>(A.u, A.irrG, A.depG, wp, R, Wo, irr, dep, A.rl);
+                col = make_float4(A.p.roughDDGIIntensity * ir.x, A.p.roughDDGIIntensity * ir.y,
+                                  A.p.roughDDGIIntensity * ir.z, 0.0f);
+            }
         } else {
-            col = skyFaces ? sample_cube4(skyFaces, A.skySize, R) : make_float4(A.sky[0], A.sky[1], A.sky[2], A.sky[3]);
+            const float ex = blue_noise(sobol, scr, x, y, int(A.p.numFrames), 0) * A.p.trim;
+            const float ey = blue_noise(sobol, scr, x, y, int(A.p.numFrames), 1) * A.p.trim;
+            const f3 Hh = importance_sample_ggx(ex, ey, n, roughness);
+            R = reflect3(mk(-Wo.x, -Wo.y, -Wo.z), Hh);
+        }
+        if (traceRay) {
+            const SdfHitTime h = trace_global_sdf<SS, FL>(sdf, A.g, wp, R, kGlobalSdfWorldSize, 0.0f, A.maxSteps);
+            hit = h.time >= 0.0f;
+            if (hit) {
+                hp = wp + R * h.time;
+                thr = A.g.cascadeVoxelSize[h.cascade] * 1.05f;
+                atlas_list(A.ad, chunks, culled, hp, list, count);
+            } else {
+                col = skyFaces ? sample_cube4(skyFaces, A.skySize, R)
+                               : make_float4(A.sky[0], A.sky[1], A.sky[2], A.sky[3]);
+            }
         }
     }
+    // eight lanes per hit: 1920x1080 with 500 objects 394 us in one lane per hit, 350 so
+    Counts c{};
+    const float4 s = sample_atlas_wave<SC, false>(A.ad, culled, objects, objInv, tiles, color, atlasDepth,
+                                                  lds[threadIdx.x >> 6], hp, mk(-R.x, -R.y, -R.z), thr, list, count, c);
+    if (hit) col = s;
+    if (!on) return;
     if (A.outHalf) Texel<__half>::st4(static_cast<__half*>(out), e, col);
     else Texel<float>::st4(static_cast<float*>(out), e, col);
 }

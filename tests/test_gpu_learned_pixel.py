@@ -148,6 +148,34 @@ def test_pass_backward_matches_the_oracle(step):
     assert np.abs(ws_).max() > 1e-3
 
 
+@pytest.mark.parametrize("W,H,radius,step,phi_normal", [(1, 1, 1, 1, 32.0), (16, 16, 2, 4, 32.0), (17, 15, 1, 8, 32.0),
+                                                        (17, 33, 2, 8, 32.0), (33, 17, 1, 2, 16.0)])
+def test_pass_backward_at_block_edges_and_both_footprints(W, H, radius, step, phi_normal):
+    """One pixel, one 16x16 block, one past it; footprints radius * step at the staged halo of 8, beyond it
+    (read directly), and the general normal exponent. Tolerances of the pass-backward test."""
+    from luxgi_amd._lib import lib
+    from luxgi_amd.ddgi import ptr, stream_handle
+    g, img, _, _ = _inputs(W, H, 21)
+    gd, gb = _gb(g)
+    tiles = np.ones(lib().luxgi_svgf_tile_count(W, H), np.uint8)
+    rng = np.random.default_rng(W + 10 * step)
+    sc = np.exp(rng.uniform(-1.0, 1.0, (H, W))).astype(np.float32)
+    go = rng.normal(size=(H, W, 4)).astype(np.float32)
+    go[..., 3] = 0.0
+    ap = abi.ReflectionAtrousParams(radius, step, 10.0, phi_normal, 1.0, 1)
+    gin = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    gsc = torch.zeros((H, W), dtype=torch.float32, device="cuda")
+    ws = torch.empty(lib().luxgi_learned_pixel_pass_backward_workspace_size(W, H), dtype=torch.uint8, device="cuda")
+    assert lib().luxgi_learned_pixel_pass_backward(C.byref(ap), W, H, C.byref(gb), ptr(_dev(tiles)), ptr(_dev(img)),
+                                                   ptr(_dev(sc)), ptr(_dev(go)), ptr(gin), ptr(gsc), ptr(ws),
+                                                   ws.numel(), stream_handle()) == 0
+    torch.cuda.synchronize()
+    wi, ws_ = oracle.learned_pixel_atrous_backward(ap, W, H, g["normals"], g["pbr"], tiles, img, sc, go)
+    a, b = gin.cpu().numpy(), gsc.cpu().numpy()
+    assert np.allclose(a, wi, rtol=1e-4, atol=1e-5 * np.abs(wi).max()), np.abs(a - wi).max()
+    assert np.allclose(b, ws_, rtol=1e-3, atol=1e-4 * np.abs(ws_).max()), np.abs(b - ws_).max()
+
+
 def test_mlp_backward_matches_the_oracle_and_is_deterministic():
     from luxgi_amd._lib import lib
     from luxgi_amd.ddgi import ptr, stream_handle

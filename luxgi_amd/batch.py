@@ -196,7 +196,7 @@ class DDGIBatch:
 
     trace="batched" (default) traces all volumes in one launch sequence over their flat ray list
     (luxgi_ddgi_trace_sdf_batched); trace="per_volume" calls luxgi_ddgi_trace_sdf per volume.
-    blend="batched" blends all volumes in one launch per map (luxgi_ddgi_probe_update_batched);
+    blend="batched" blends both maps of all volumes in one launch (luxgi_ddgi_probe_update_batched);
     blend="per_volume" calls luxgi_ddgi_probe_update per volume; "auto" (default) takes the batched
     form when every volume fits it. With `streams` > 0 the per-volume work is spread over that many
     side streams (default priority), forked from and joined to the current stream."""

@@ -362,7 +362,7 @@ __global__ void border_kernel(SA* __restrict__ atlas, int W, int n, int pxy, int
 // MFMA form. With shared ray directions the blend of a block of 16 probes is
 //   depth: C[Td x 16] = W_d[Td x R] . B_r[R x 16]  and  W_d . B_r2   (probe g, r and r^2)
 //   irr:   C[Ti x 16] = W_i[Ti x R] . B_c[R x 16]  for c = R, G, B
-// contracted on the 16x16x32 MFMA (probe_blend_map_kernel below), one map per launch. The
+// contracted on the 16x16x32 MFMA (blend_map_block below), one map per block. The
 // epilogue normalises by 1/(2 S[t]), applies the gamma, stages the interiors in LDS and writes
 // each probe's full bordered tile with the hysteresis blend. A probe whose staged directions
 // differ from ray row 0 is flagged; probe_update_kernel then recomputes the flagged probes with
@@ -486,13 +486,12 @@ __device__ __forceinline__ floatx4 mfma_lp(V ah, V al, V bh, V bl, floatx4 acc) 
 }
 
 // ---------------------------------------------------------------------------
-// The same contraction with one map per launch (MAP 0: depth moments r, r^2; MAP 1: irradiance
+// The same contraction with one map per block (MAP 0: depth moments r, r^2; MAP 1: irradiance
 // R, G, B), as the reference dispatches DepthProbeUpdate.comp and IrradianceProbeUpdate.comp
-// separately (DDGIRenderer.cpp:347-375). Each launch holds only its own map's accumulators and
-// stages only its own output tile in LDS (depth 32 KB, irradiance 16 KB), so four 256-lane blocks
-// fit a CU and the 1,024 blocks of a 16,384-probe volume are resident at once. The depth launch
-// reads only the direction/distance rays and checks the directions against row 0; the irradiance
-// launch reads only the radiance rays (and the directions too when the depth map is not
+// separately (DDGIRenderer.cpp:347-375). A block holds only its own map's accumulators and stages
+// only its own output tile in LDS (depth 32 KB, irradiance 16 KB), so four 256-lane blocks fit a CU.
+// The depth map reads only the direction/distance rays and checks the directions against row 0; the
+// irradiance map reads only the radiance rays (and the directions too when the depth map is not
 // updated in the same call, CHECK).
 // ---------------------------------------------------------------------------
 constexpr int kWB = 4;  // previous-atlas loads each lane keeps in flight in the tile writer
@@ -758,6 +757,33 @@ __global__ __launch_bounds__(256, 4) void probe_blend_map_kernel(
                                                   mismatch, tpad, Rpad, lds, sMis);
 }
 
+// Both maps in one launch: the first half of the grid blends depth (the longer chain), the second half
+// irradiance. A map's time is one block's chain of ray chunks and tile rows, and up to 8,192 probes
+// leave half the chip free for the other map: whole updates 38 -> 25 us at 8x8x8x64, 68 -> 49 at
+// 16x16x16x256, 107 -> 105 at 32x16x32x256, where the irradiance blocks fill in as depth blocks end.
+template <class T>
+union MapsLds {
+    MapLds<0, T> depth;
+    MapLds<1, T> irr;
+};
+template <class SR, class SA, class T, bool SPLIT>
+__global__ __launch_bounds__(256, 4) void probe_blend_maps_kernel(
+    UpdateArgs A, const SR* __restrict__ radiance, const SR* __restrict__ dirDist, const SA* __restrict__ prevI,
+    const SA* __restrict__ prevD, SA* __restrict__ outI, SA* __restrict__ outD, const float* __restrict__ dirs0,
+    const T* __restrict__ Wih, const T* __restrict__ Wil, const float* __restrict__ Sih, const T* __restrict__ Wdh,
+    const T* __restrict__ Wdl, const float* __restrict__ Sdh, uint8_t* __restrict__ mismatch, int tpI, int tpD,
+    int Rpad) {
+    __shared__ MapsLds<T> lds;
+    __shared__ int sMis[kMG];
+    const int groups = gridDim.x / 2;
+    if ((int)blockIdx.x < groups)
+        blend_map_block<SR, SA, T, SPLIT, 0, false>(A, blockIdx.x * kMG, radiance, dirDist, prevD, outD, dirs0, Wdh, Wdl,
+                                                    Sdh, mismatch, tpD, Rpad, lds.depth, sMis);
+    else
+        blend_map_block<SR, SA, T, SPLIT, 1, false>(A, (blockIdx.x - groups) * kMG, radiance, dirDist, prevI, outI,
+                                                    dirs0, Wih, Wil, Sih, mismatch, tpI, Rpad, lds.irr, sMis);
+}
+
 // ---------------------------------------------------------------------------
 // Several volumes in one launch per pass (no counterpart in the reference, which dispatches the
 // update per volume): each volume's arguments and workspace pointers in a device descriptor, the
@@ -830,6 +856,29 @@ __global__ __launch_bounds__(256, 4) void probe_blend_map_batched_kernel(const U
                                                     static_cast<const SA*>(D.prevI), static_cast<SA*>(D.outI), D.dirs0,
                                                     static_cast<const T*>(D.Wih), static_cast<const T*>(D.Wil), D.Sih,
                                                     D.mismatch, D.tpI, D.Rp, lds, sMis);
+}
+
+// both maps in one launch, as probe_blend_maps_kernel
+template <class SR, class SA, class T, bool SPLIT>
+__global__ __launch_bounds__(256, 4) void probe_blend_maps_batched_kernel(const UpdateVolumeDesc* __restrict__ d, int n) {
+    __shared__ MapsLds<T> lds;
+    __shared__ int sMis[kMG];
+    const int groups = gridDim.x / 2;
+    const bool depth = (int)blockIdx.x < groups;
+    const int group = depth ? blockIdx.x : blockIdx.x - groups;
+    const UpdateVolumeDesc& D = d[batch_update_volume(d, n, group)];
+    const int p0 = (group - D.groupStart) * kMG;
+    if (p0 >= D.A.P) return;  // uniform per block
+    if (depth)
+        blend_map_block<SR, SA, T, SPLIT, 0, false>(D.A, p0, static_cast<const SR*>(D.rad), static_cast<const SR*>(D.dd),
+                                                    static_cast<const SA*>(D.prevD), static_cast<SA*>(D.outD), D.dirs0,
+                                                    static_cast<const T*>(D.Wdh), static_cast<const T*>(D.Wdl), D.Sdh,
+                                                    D.mismatch, D.tpD, D.Rp, lds.depth, sMis);
+    else
+        blend_map_block<SR, SA, T, SPLIT, 1, false>(D.A, p0, static_cast<const SR*>(D.rad), static_cast<const SR*>(D.dd),
+                                                    static_cast<const SA*>(D.prevI), static_cast<SA*>(D.outI), D.dirs0,
+                                                    static_cast<const T*>(D.Wih), static_cast<const T*>(D.Wil), D.Sih,
+                                                    D.mismatch, D.tpI, D.Rp, lds.irr, sMis);
 }
 
 // the per-probe fix-up of flagged probes (directions not those of row 0), 4 probes at a time
@@ -961,19 +1010,20 @@ static int launch_maps(const UpdateArgs& A, const SR* rad, const SR* dd, const S
         LUXGI_LAUNCH_CHECK();
     }
     const dim3 grid((A.P + kMG - 1) / kMG);
+    if (A.doDepth && A.doIrr) {
+        hipLaunchKernelGGL((probe_blend_maps_kernel<SR, SA, T, SPLIT>), dim3(2 * grid.x), dim3(256), 0, st, A, rad, dd,
+                           pI, pD, oI, oD, dirs0, Wih, Wil, w.Sih, Wdh, Wdl, w.Sdh, w.mismatch, tpI, tpD, Rp);
+        LUXGI_LAUNCH_CHECK();
+        return LUXGI_OK;
+    }
     if (A.doDepth) {
         hipLaunchKernelGGL((probe_blend_map_kernel<SR, SA, T, SPLIT, 0, false>), grid, dim3(256), 0, st, A, rad, dd, pD,
                            oD, dirs0, Wdh, Wdl, w.Sdh, w.mismatch, tpD, Rp);
         LUXGI_LAUNCH_CHECK();
     }
-    if (A.doIrr) {
-        // the directions were checked by the depth launch; alone, this launch checks them
-        if (A.doDepth)
-            hipLaunchKernelGGL((probe_blend_map_kernel<SR, SA, T, SPLIT, 1, false>), grid, dim3(256), 0, st, A, rad, dd,
-                               pI, oI, dirs0, Wih, Wil, w.Sih, w.mismatch, tpI, Rp);
-        else
-            hipLaunchKernelGGL((probe_blend_map_kernel<SR, SA, T, SPLIT, 1, true>), grid, dim3(256), 0, st, A, rad, dd,
-                               pI, oI, dirs0, Wih, Wil, w.Sih, w.mismatch, tpI, Rp);
+    if (A.doIrr) {  // alone, the irradiance map checks the directions
+        hipLaunchKernelGGL((probe_blend_map_kernel<SR, SA, T, SPLIT, 1, true>), grid, dim3(256), 0, st, A, rad, dd, pI,
+                           oI, dirs0, Wih, Wil, w.Sih, w.mismatch, tpI, Rp);
         LUXGI_LAUNCH_CHECK();
     }
     return LUXGI_OK;
@@ -1223,20 +1273,16 @@ static int launch_batched(const LuxgiUpdateBatch& b, const UpdateVolumeDesc* d, 
     hipLaunchKernelGGL(weights_batched_kernel<T>, dim3(b.maxWeightBlocks, b.count, 2), dim3(256), 0, st, d,
                        SPLIT ? 1 : 0);
     LUXGI_LAUNCH_CHECK();
-    if (doDepth) {
+    if (doDepth && doIrr)
+        hipLaunchKernelGGL((probe_blend_maps_batched_kernel<SR, SA, T, SPLIT>), dim3(2 * b.groups), dim3(256), 0, st, d,
+                           b.count);
+    else if (doDepth)
         hipLaunchKernelGGL((probe_blend_map_batched_kernel<SR, SA, T, SPLIT, 0, false>), dim3(b.groups), dim3(256), 0,
                            st, d, b.count);
-        LUXGI_LAUNCH_CHECK();
-    }
-    if (doIrr) {
-        if (doDepth)
-            hipLaunchKernelGGL((probe_blend_map_batched_kernel<SR, SA, T, SPLIT, 1, false>), dim3(b.groups), dim3(256),
-                               0, st, d, b.count);
-        else
-            hipLaunchKernelGGL((probe_blend_map_batched_kernel<SR, SA, T, SPLIT, 1, true>), dim3(b.groups), dim3(256),
-                               0, st, d, b.count);
-        LUXGI_LAUNCH_CHECK();
-    }
+    else if (doIrr)
+        hipLaunchKernelGGL((probe_blend_map_batched_kernel<SR, SA, T, SPLIT, 1, true>), dim3(b.groups), dim3(256), 0,
+                           st, d, b.count);
+    LUXGI_LAUNCH_CHECK();
     hipLaunchKernelGGL((fixup_batched_kernel<SR, SA>), dim3(b.groups), dim3(256), 0, st, d, b.count);
     LUXGI_LAUNCH_CHECK();
     return LUXGI_OK;

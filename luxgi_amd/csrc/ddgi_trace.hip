@@ -58,6 +58,7 @@ struct TraceArgs {
     int maxSteps, P, R, rayWidth;
     float hitEps;
     int fineLayout;                // LuxgiLayout of the fine volume (the kernels' template argument)
+    int waveRays;                  // rays per wave: 64, or 16 where few rays leave the chip idle
     LuxgiTraceVolume vol;          // the volume of a single-volume call
     const LuxgiTraceVolume* vols;  // the volumes of a batched call (device memory), their count
     int nVols;                     // and the total of their rays
@@ -359,16 +360,23 @@ __device__ __forceinline__ bool find_ray(const TraceArgs& A, long long gid, cons
     }
 }
 
+// Flat lane of this thread's ray: each wave has A.waveRays of them, one per lane from lane 0.
+__device__ __forceinline__ bool lane_traces(const TraceArgs& A) { return (int)(threadIdx.x & 63) < A.waveRays; }
+__device__ __forceinline__ long long wave_ray(const TraceArgs& A) {
+    const int lane = threadIdx.x & 63;
+    return (xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6)) * A.waveRays + min(lane, A.waveRays - 1);
+}
+
 // Sphere trace of one ray per lane.
 template <class SS, class SR, bool COUNT, int FL, int MODE>
 __global__ __launch_bounds__(256) void march_kernel(TraceArgs A, float4* __restrict__ recA, uint8_t* __restrict__ recC,
                                                     unsigned long long* __restrict__ counters) {
-    const long long gid = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const long long gid = wave_ray(A);
     unsigned long long cMip = 0, cFine = 0, cSteps = 0, cHits = 0;
     const LuxgiTraceVolume* v;
     int probe, ray;
     size_t rid;
-    if (find_ray<MODE>(A, gid, v, probe, ray, rid))
+    if (find_ray<MODE>(A, gid, v, probe, ray, rid) && lane_traces(A))
         march_ray<SS, SR, COUNT, FL>(A, MODE == 2 ? A.scenes[v->scene] : A.scene, *v, probe, ray, rid, recA, recC, cMip,
                                      cFine, cSteps, cHits);
     if (COUNT) {
@@ -403,12 +411,12 @@ __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __
                                                     const float4* __restrict__ recA, const uint8_t* __restrict__ recC,
                                                     unsigned long long* __restrict__ counters) {
     __shared__ AtlasQueryLds lds[4];
-    const long long gid = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const long long gid = wave_ray(A);
     Counts c = {0, 0, 0, 0, 0, 0, 0};
     const LuxgiTraceVolume* v;
     int probe, ray;
     size_t rid;
-    const bool valid = find_ray<MODE>(A, gid, v, probe, ray, rid);
+    const bool valid = find_ray<MODE>(A, gid, v, probe, ray, rid) && lane_traces(A);
     const TraceScene& S = MODE == 2 ? A.scenes[v->scene] : A.scene;
     float4 ra = make_float4(-1.f, 0.f, 0.f, 0.f);
     if (valid) ra = recA[rid];
@@ -499,12 +507,19 @@ extern "C" size_t luxgi_ddgi_trace_workspace_size(const LuxgiDDGIUniform* u, int
     return trace_workspace_layout(P * R, objectCapacity, nullptr, nullptr);
 }
 
+// Up to this many rays a wave takes 16 of them. A small trace is the chain of its longest rays and of its
+// waves' hits, eight at a time, with most of the chip idle: shorter waves spread the hits over four
+// times as many. 4,096 rays 86 -> 66 us, 32,768 87 -> 67, 65,536 92 -> 82; 100,100 rays already
+// lose by it (64 -> 75) and 196,608 more (74 -> 94).
+constexpr long long kFewRays = 65536;
+
 // The kernels of one trace: object inverses, march, shade. MODE 0: one volume, 1: a batch over A.scene,
 // 2: a batch over per-volume scenes (A.scenes, nScenes of them, at most maxObjects objects each).
 template <class SS, class SC, class SR, bool COUNT, int MODE>
-static int launch_trace(const TraceArgs& A, int nScenes, int maxObjects, const TraceWorkspace& w,
+static int launch_trace(TraceArgs A, int nScenes, int maxObjects, const TraceWorkspace& w,
                         unsigned long long* counters, hipStream_t st) {
     const long long lanes = MODE != 0 ? A.totalRays : (long long)A.P * ((A.R + 63) & ~63);
+    A.waveRays = lanes <= kFewRays ? 16 : 64;
     if (MODE == 2) {
         if (maxObjects > 0) {
             hipLaunchKernelGGL(trace_prepare_scenes_kernel, dim3((maxObjects + 255) / 256, nScenes), dim3(256), 0, st,
@@ -516,7 +531,7 @@ static int launch_trace(const TraceArgs& A, int nScenes, int maxObjects, const T
                            st, A.scene.objects, A.scene.objectCapacity, w.inv);
         LUXGI_LAUNCH_CHECK();
     }
-    const dim3 grid((int)((lanes + 255) / 256));
+    const dim3 grid((int)((lanes + 4 * A.waveRays - 1) / (4 * A.waveRays)));
     if (A.fineLayout == LUXGI_LAYOUT_BRICK4)
         hipLaunchKernelGGL((march_kernel<SS, SR, COUNT, LUXGI_LAYOUT_BRICK4, MODE>), grid, dim3(256), 0, st, A, w.recA,
                            w.recC, counters);

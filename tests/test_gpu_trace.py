@@ -107,6 +107,26 @@ def test_trace_shade_groups_at_wave_and_list_edges(rays):
     assert lit.mean() > 0.1
 
 
+@pytest.mark.parametrize("rays", [64, 37])
+def test_trace_is_the_same_for_short_and_full_waves(rays):
+    """Up to 65,536 padded rays a wave takes 16 of them, above that 64: a volume of 1,024 probes and one of
+    32 more with the same first 1,024 give the same texels there, bit for bit, whole and partial waves."""
+    from luxgi_amd.ddgi import DDGIVolume, DeviceScene
+    prims, sdf, mip, g, atlas = _scenes.small_scene()
+    ds = DeviceScene(g, sdf, mip, atlas)
+    p = _scenes.trace_params(rot_seed=23)
+    outs = []
+    for ny in (32, 33):
+        u = abi.make_uniform((32, ny, 1), (-0.9, -0.9, 0.1), (1.8 / 32, 1.8 / 32, 1.0), rays)
+        vol = DDGIVolume(u, flags_buffer=True)
+        vol.trace_rays(ds, p)
+        torch.cuda.synchronize()
+        outs.append([t[:1024].cpu().numpy() for t in (vol.radiance, vol.dir_dist, vol.ray_flags)])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    assert (outs[0][2] == 1).mean() > 0.3
+
+
 def test_trace_unorm8_atlas_and_offsets():
     prims, sdf, mip, g, atlas = _scenes.small_scene(color_storage=abi.STORAGE_UNORM8)
     u = _scenes.small_uniform(rays=96, counts=(5, 4, 6))

@@ -427,4 +427,19 @@ __device__ __forceinline__ int2 xcd_block_2d() {
     return make_int2(int(t % gridDim.x), int(t / gridDim.x));
 }
 
+// The pixel of a lane in a launch of one-wave blocks of 8x8 pixels whose cost varies over the image: the XCDs
+// take 32x32-pixel squares in turn (16 blocks each), which keeps a square's lookups in one L2 and, unlike the
+// bands above, deals the costly parts of the image to all XCDs. Blocks of the last squares lie outside.
+inline dim3 xcd_square_grid(int W, int H) {
+    const long long squares = (long long)((W + 31ll) / 32) * ((H + 31ll) / 32), groups = (squares + kXcds - 1) / kXcds;
+    const long long y = groups < 65535 ? groups : 65535;
+    return dim3(16 * kXcds, unsigned(y), unsigned((groups + y - 1) / y));
+}
+__device__ __forceinline__ uint2 xcd_square_pixel(int W) {
+    const uint32_t square = (blockIdx.z * gridDim.y + blockIdx.y) * kXcds + (blockIdx.x & (kXcds - 1));
+    const uint32_t perRow = ((uint32_t)W + 31) / 32, block = blockIdx.x / kXcds;
+    return make_uint2((square % perRow) * 32 + (block & 3) * 8 + (threadIdx.x & 7),
+                      (square / perRow) * 32 + (block >> 2) * 8 + (threadIdx.x >> 3));
+}
+
 }  // namespace luxgi

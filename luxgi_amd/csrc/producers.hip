@@ -146,8 +146,12 @@ __device__ __forceinline__ f3 importance_sample_ggx(float ex, float ey, f3 N, fl
 
 __device__ __forceinline__ f3 reflect3(f3 I, f3 N) { return I - N * (2.0f * dot3(N, I)); }
 
+// Bound by the divergent march and atlas lookups. One wave per block: a block then ends with its own longest
+// ray and not with that of four waves, and 8x8 pixels send more alike rays than 16x4. The order of the blocks
+// is xcd_square_pixel's. 1920x1080, 500 objects: 346 us in 16x16 blocks in launch order, 333 in one-wave
+// blocks, 323 in 32x32 squares (16x16: 333, 64x64: 327; a band of rows per XCD: 349).
 template <class SS, int FL, class SC, class SA>
-__global__ __launch_bounds__(256) void reflection_kernel(ReflArgsP A, const float* __restrict__ normals,
+__global__ __launch_bounds__(64) void reflection_kernel(ReflArgsP A, const float* __restrict__ normals,
                                                          const float* __restrict__ pbr, const float* __restrict__ depth,
                                                          const uint8_t* __restrict__ sobol,
                                                          const uint8_t* __restrict__ scr, SdfView<SS> sdf,
@@ -160,10 +164,11 @@ __global__ __launch_bounds__(256) void reflection_kernel(ReflArgsP A, const floa
                                                          const float* __restrict__ skyFaces,
                                                          const SA* __restrict__ irr, const SA* __restrict__ dep,
                                                          void* __restrict__ out) {
-    __shared__ AtlasQueryLds lds[4];
-    const int x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 16 + (threadIdx.x >> 4);
-    const size_t e = (size_t)y * A.W + x;
-    const float d = x < A.W && y < A.H ? depth[e] : 1.0f;
+    __shared__ AtlasQueryLds lds;
+    const uint2 px = xcd_square_pixel(A.W);
+    const int x = int(px.x), y = int(px.y);
+    const size_t e = (size_t)px.y * A.W + px.x;
+    const float d = px.x < (uint32_t)A.W && px.y < (uint32_t)A.H ? depth[e] : 1.0f;
     const bool on = d != 1.0f;  // sky: the reference leaves the texel as it was
     float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
     f3 hp = mk(0.f, 0.f, 0.f), R = hp;
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(256) void reflection_kernel(ReflArgsP A, const floa
     // eight lanes per hit: 1920x1080 with 500 objects 394 us in one lane per hit, 350 so
     Counts c{};
     const float4 s = sample_atlas_wave<SC, false>(A.ad, culled, objects, objInv, tiles, color, atlasDepth,
-                                                  lds[threadIdx.x >> 6], hp, mk(-R.x, -R.y, -R.z), thr, list, count, c);
+                                                  lds, hp, mk(-R.x, -R.y, -R.z), thr, list, count, c);
     if (hit) col = s;
     if (!on) return;
     if (A.outHalf) Texel<__half>::st4(static_cast<__half*>(out), e, col);
@@ -282,7 +287,7 @@ template <class SS, int FL, class SC, class SA>
 static void launch_reflection(const ReflArgsP& A, const LuxgiGBuffer* gb, const LuxgiBlueNoise* nz,
                               const LuxgiSDFVolume* vol, const LuxgiSurfaceAtlas* at, const float* inv,
                               const float* skyFaces, const LuxgiProbeAtlas* probes, void* out, hipStream_t st) {
-    hipLaunchKernelGGL((reflection_kernel<SS, FL, SC, SA>), dim3((A.W + 15) / 16, (A.H + 15) / 16), dim3(256), 0, st,
+    hipLaunchKernelGGL((reflection_kernel<SS, FL, SC, SA>), xcd_square_grid(A.W, A.H), dim3(64), 0, st,
                        A, gb->normals, gb->pbr, gb->depth, nz->sobol, nz->scrambling, sdf_view<SS>(vol), at->chunks,
                        at->culledObjects, at->objects, inv, at->tiles, static_cast<const SC*>(at->color), at->depth,
                        skyFaces, probes ? static_cast<const SA*>(probes->irradiance) : nullptr,

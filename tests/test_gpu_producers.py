@@ -140,3 +140,39 @@ def test_sdf_reflection_matches_oracle(layout, atlas_layout):
     assert ok.mean() >= 0.99, ok.mean()
     hit = (want[..., 3] > 0) & (want[..., 3] != 1.0)
     assert hit[~sky_px].mean() > 0.2  # rays that read the atlas
+
+
+@pytest.mark.parametrize("W,H", [(1, 1), (1, 300), (300, 1), (31, 33), (32, 256), (257, 40), (289, 95)])
+def test_sdf_reflection_traces_every_pixel_once_at_the_edges_of_its_pixel_squares(W, H):
+    """Mirror rays over images below, at and past the 8x8 blocks, the 32x32 squares and the rows of eight of
+    them: pixels that are not sky agree with the oracle (the bounds of the test above; at least two
+    pixels may graze past a surface), sky pixels and the texels after the image keep their value."""
+    from luxgi_amd.ddgi import DeviceScene, to_device
+    from luxgi_amd.producers import BlueNoiseTables, sdf_reflection
+    from luxgi_amd.svgf import make_gbuffer
+    prims, sdf, mip, g, atlas = _scenes.small_scene()
+    VP, VPp, eye, _ = scene.camera_pair(64, 64, seed=9, eye=(0.1, 0.3, 0.75))
+    VPI = np.linalg.inv(VP)
+    prims_dev = to_device(np.frombuffer(prims.tobytes(), dtype=np.uint8))
+    gb, _, _ = make_gbuffer(prims_dev, len(prims), g, torch.from_numpy(sdf).cuda(), 64, VPI, VPp, W, H, seed=3,
+                            with_mask=False)
+    gb["pbr"][..., 1] = 0.01  # mirror
+    normals, pbr, depth = (gb[k].cpu().numpy() for k in ("normals", "pbr", "depth"))
+    rng = np.random.default_rng(W * 1000 + H)
+    sky = rng.uniform(0.0, 2.0, size=(6, 8, 8, 4)).astype(np.float32)
+    ds = DeviceScene(g, sdf, mip, atlas, layout=abi.LAYOUT_CELL8, sky_faces=sky, sky_size=8)
+    sobol, scr = _noise(2)
+    p = abi.SdfReflectionParams()
+    p.trim, p.numFrames = 0.9, 17
+    p.cameraPosition[:] = [eye[0], eye[1], eye[2], 1.0]
+    p.viewProjInv = abi.mat4_colmajor(VPI)
+    whole = torch.full((W * H + 4096, 4), -5.0, dtype=torch.float32, device="cuda")
+    sdf_reflection(p, BlueNoiseTables(sobol, scr), gb, ds, whole[: W * H].view(H, W, 4))
+    torch.cuda.synchronize()
+    got = whole[: W * H].view(H, W, 4).cpu().numpy()
+    want = oracle.sdf_reflection(p, sobol, scr, W, H, normals, pbr, depth, g, sdf, mip, 64, 16, atlas, sky_faces=sky,
+                                 sky_size=8, out=np.full((H, W, 4), -5.0))
+    sky_px = depth == 1.0
+    assert np.all(got[sky_px] == -5.0) and bool((whole[W * H:] == -5.0).all())
+    ok = np.all(np.abs(got - want) <= 2e-3 * (1 + np.abs(want)), axis=-1)[~sky_px]
+    assert (~ok).sum() <= max(2, 0.01 * ok.size), ((~ok).sum(), ok.size)

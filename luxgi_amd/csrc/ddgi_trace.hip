@@ -67,11 +67,7 @@ struct TraceArgs {
 
 // ---------------------------------------------------------------------------
 // March (tracyGlobalSDF, SDFCommon.glsl:98-194): one lane per ray, the 64 lanes
-// of a wave on 64 rays of one probe. Blocks are mapped to probes XCD by XCD:
-// the dispatcher deals blocks to the 8 XCDs round-robin, so block b runs on XCD
-// b % 8; the mapping gives each XCD a contiguous range of rays (a slab of
-// probes) that it walks in order, which keeps the SDF lines its rays touch in
-// its own L2. A front hit's record (hitTime, texture UV of the hit step; cascade)
+// of a wave on 64 rays of one probe, in trace_block's order. A front hit's record (hitTime, texture UV of the hit step; cascade)
 // goes to the workspace for shade_kernel.
 // ---------------------------------------------------------------------------
 
@@ -360,11 +356,29 @@ __device__ __forceinline__ bool find_ray(const TraceArgs& A, long long gid, cons
     }
 }
 
+// The block of rays of a launched block. The dispatcher deals blocks to the 8 XCDs in turn (block b runs on
+// XCD b % 8). Each XCD takes kXcdRun blocks in a row (65,536 rays; 256 probes of 256 rays), whose SDF lines
+// stay in its L2, and the next run lies 8 runs on, so at any time the XCDs walk neighbouring probes and share
+// what they read from the memory side. With one eighth of the volume per XCD they walk eight distant slabs
+// and end unevenly: 32x16x32 probes x 256 rays 1,518 us against 1,350 (runs of 8, 32, 128, 512, 1,024 blocks:
+// 1,445, 1,455, 1,482, 1,355, 1,394; probes in 4^3 or 8^3 cubes: 1,444, 1,369). The blocks after the last
+// whole turn go in eighths, and so does a launch below two turns (1,048,576 rays): 32x8x16x144 in FP16, one turn
+// and a half, 124 us in eighths against 130, 13x7x11x100 68 against 70 undealt; from two turns on runs are the
+// faster, 16x16x16x256 441 -> 420, 17x9x31x256 linear FP16 366 -> 346, 32x32x32x64 linear 675 -> 609.
+constexpr int kXcdRun = 256;
+__device__ __forceinline__ long long trace_block() {
+    constexpr uint32_t turn = kXcds * kXcdRun;
+    const uint32_t b = blockIdx.x, whole = gridDim.x < 2 * turn ? 0 : gridDim.x / turn * turn;
+    if (b >= whole) return whole + xcd_block(b - whole, gridDim.x - whole);
+    const uint32_t r = b % turn;
+    return b - r + r % kXcds * kXcdRun + r / kXcds;
+}
+
 // Flat lane of this thread's ray: each wave has A.waveRays of them, one per lane from lane 0.
 __device__ __forceinline__ bool lane_traces(const TraceArgs& A) { return (int)(threadIdx.x & 63) < A.waveRays; }
 __device__ __forceinline__ long long wave_ray(const TraceArgs& A) {
     const int lane = threadIdx.x & 63;
-    return (xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6)) * A.waveRays + min(lane, A.waveRays - 1);
+    return (trace_block() * 4 + (threadIdx.x >> 6)) * A.waveRays + min(lane, A.waveRays - 1);
 }
 
 // Sphere trace of one ray per lane.

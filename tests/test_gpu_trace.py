@@ -127,6 +127,30 @@ def test_trace_is_the_same_for_short_and_full_waves(rays):
     assert (outs[0][2] == 1).mean() > 0.3
 
 
+@pytest.mark.parametrize("nz", [17, 25])
+def test_trace_is_the_same_for_blocks_dealt_in_runs_and_in_eighths(nz):
+    """From 4,096 blocks of 256 padded rays on the XCDs take runs of 256 blocks, below that, and after the last
+    whole turn of 2,048, eighths. A volume past that line (one and two turns with a ragged tail) gives the texels
+    of its first and its last 16 layers, each traced below it, bit for bit; the probe positions are exact
+    binary fractions, so the parts see the same origins."""
+    from luxgi_amd.ddgi import DDGIVolume, DeviceScene
+    prims, sdf, mip, g, atlas = _scenes.small_scene()
+    ds = DeviceScene(g, sdf, mip, atlas)
+    p = _scenes.trace_params(rot_seed=29)
+
+    def trace(z0, n):
+        u = abi.make_uniform((31, 33, n), (-0.5, -0.5, -0.5 + z0 / 32), (1 / 32, 1 / 32, 1 / 32), 37)
+        vol = DDGIVolume(u, flags_buffer=True)
+        vol.trace_rays(ds, p)
+        torch.cuda.synchronize()
+        return [t.cpu().numpy()[: 31 * 33 * n] for t in (vol.radiance, vol.dir_dist, vol.ray_flags)]
+
+    whole, first, last = trace(0, nz), trace(0, 16), trace(nz - 16, 16)
+    for w, a, b in zip(whole, first, last):
+        assert np.array_equal(w[: len(a)], a) and np.array_equal(w[-len(b):], b)
+    assert (whole[2] == 1).mean() > 0.05
+
+
 def test_trace_unorm8_atlas_and_offsets():
     prims, sdf, mip, g, atlas = _scenes.small_scene(color_storage=abi.STORAGE_UNORM8)
     u = _scenes.small_uniform(rays=96, counts=(5, 4, 6))

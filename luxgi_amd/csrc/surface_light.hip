@@ -50,15 +50,26 @@ __device__ __forceinline__ float4 bilinear_rgba(const S* __restrict__ img, int W
                        lerp2(a.w, b.w, c.w, d.w));
 }
 
-// BRDF (Raytraced/BRDF.glsl:12-79, the 7-argument form)
-__device__ __forceinline__ f3 brdf_ggx(f3 albedo, f3 n, float rough, float metal, f3 view, f3 h, f3 l) {
+// a . b with the fused products named. Near a mirror the BRDF divides by the square of cosLh^2 (a^2 - 1) + 1,
+// which turns the last bit of the half vector's length into percents of the highlight: left to the compiler,
+// the product that is rounded first, and with it the texel, depends on the code around the call.
+__device__ __forceinline__ float dot_named(f3 a, f3 b) {
+    return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y));
+}
+
+// BRDF (Raytraced/BRDF.glsl:12-79, the 7-argument form, the half vector worked out here)
+__device__ __forceinline__ f3 brdf_ggx(f3 albedo, f3 n, float rough, float metal, f3 view, f3 l) {
+    const f3 s = l + view;
+    const float len = sqrtf(dot_named(s, s));
+    const f3 h = mk(s.x / len, s.y / len, s.z / len);
     const f3 F0 = mk(mixf(0.04f, albedo.x, metal), mixf(0.04f, albedo.y, metal), mixf(0.04f, albedo.z, metal));
-    const float cosLi = fmaxf(0.0f, dot3(n, l)), cosLh = fmaxf(0.0f, dot3(n, h)), NdotV = fmaxf(0.0f, dot3(n, view));
-    const float c = clampf(1.0f - fmaxf(dot3(h, view), 0.0f), 0.0f, 1.0f);
+    const float cosLi = fmaxf(0.0f, dot_named(n, l)), cosLh = fmaxf(0.0f, dot_named(n, h));
+    const float NdotV = fmaxf(0.0f, dot_named(n, view));
+    const float c = clampf(1.0f - fmaxf(dot_named(h, view), 0.0f), 0.0f, 1.0f);
     const float c5 = c * c * c * c * c;
     const f3 F = mk(F0.x + (1.0f - F0.x) * c5, F0.y + (1.0f - F0.y) * c5, F0.z + (1.0f - F0.z) * c5);
     const float alpha = rough * rough, a2 = alpha * alpha;
-    const float denom = cosLh * cosLh * (a2 - 1.0f) + 1.0f;
+    const float denom = __builtin_fmaf(cosLh * cosLh, a2 - 1.0f, 1.0f);
     const float D = a2 / (kPiF * denom * denom);
     const float r = rough + 1.0f, k = r * r * 0.125f;
     const float G = cosLi / (cosLi * (1.0f - k) + k) * (NdotV / (NdotV * (1.0f - k) + k));
@@ -235,9 +246,8 @@ __global__ __launch_bounds__(256, 4) void surface_light_kernel(SurfaceArgs A, co
                     const float inten = __powf(sm.lights[l].intensity, 1.4f) + 0.1f;
                     const float* lc = sm.lights[l].color;
                     const f3 Lrad = mk(lc[0] * inten, lc[1] * inten, lc[2] * inten);
-                    const f3 Lh = normalize3(L + view);
                     const float cosLi = fmaxf(0.0f, dot3(n, L));
-                    const f3 b = brdf_ggx(mk(cc.x, cc.y, cc.z), n, pbr.y, pbr.x, view, Lh, L);
+                    const f3 b = brdf_ggx(mk(cc.x, cc.y, cc.z), n, pbr.y, pbr.x, view, L);
                     const float s = cosLi * shadow * atten;
                     acc = acc + mk(b.x * Lrad.x * s, b.y * Lrad.y * s, b.z * Lrad.z * s);
                 }

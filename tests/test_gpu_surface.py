@@ -172,6 +172,70 @@ def test_direct_light_at_the_edges_of_the_texel_chunks_and_light_groups(tile, n_
     assert np.abs(want[..., :3]).max() > 0.05
 
 
+def _fma32(a, b, c):
+    """a b + c rounded to FP32 (the product is exact in FP64)."""
+    return np.float32(float(a) * float(b) + float(c))
+
+
+def test_near_mirror_highlight_rounds_its_half_vector_in_one_stated_order():
+    """The highlight of a roughness of 10 / 255 divides by cos^2 (a^2 - 1) + 1 with a^2 = 2.4e-6, so the last
+    bit of the half vector's length moves the texel by percents. One directional light around the normal of a
+    constant G-buffer (world position 0, normal and view +x: every dot product with them is exact); the length
+    is sqrt(fma(z, z, fma(x, x, y y))), and the lights are those for which rounding x x first gives a highlight
+    at least 2% away. Expected in FP64 from that FP32 length and denominator; the remaining operations are FP32
+    with fewer than 30 roundings of 6e-8, none cancelling: 1e-4 leaves room for the intensity's fast power."""
+    from luxgi_amd.ddgi import DeviceScene, to_device
+    from luxgi_amd.surface import SurfaceCache
+    f = np.float32
+    _, _, _, g, _ = _scenes.small_scene()
+    atlas = scene.build_atlas(scene.scene_small(seed=1), resolution=256, tile=8, seed=3, threshold=0.05,
+                              surface_gbuffer=True)
+    atlas.gb_color[...] = 0.5
+    atlas.gb_color[..., 3] = 0.0
+    atlas.gb_normal[...] = 0.0
+    atlas.gb_normal[..., 0] = 1.0
+    atlas.gb_pbr[...] = 0
+    atlas.gb_pbr[..., 1] = 10
+    ds = DeviceScene(g, np.ones((64, 64, 64), np.float32), np.ones((16, 16, 16), np.float32), atlas)
+    sc = SurfaceCache(atlas, out_storage=abi.STORAGE_FP32)
+    a2 = f((10 / 255) ** 4)
+
+    def light_of(L, first):
+        x, y, z = f(L[0] + f(1)), L[1], L[2]
+        inner = _fma32(x, x, f(y * y)) if first else _fma32(y, y, f(x * x))
+        c = f(x / np.sqrt(_fma32(z, z, inner)))
+        denom = float(_fma32(f(c * c), f(a2 - f(1)), 1.0))
+        rough, li, lv = 10 / 255, float(L[0]), float(c)
+        fr = 0.04 + 0.96 * (1.0 - lv) ** 5
+        k = (rough + 1) ** 2 * 0.125
+        G = li / (li * (1 - k) + k) * (1 / ((1 - k) + k))
+        spec = float(a2) / (np.pi * denom * denom) * G / (4 * li)
+        return ((1 - fr) / np.pi * 0.5 + fr * spec) * (1.0 ** 1.4 + 0.1) * li
+
+    rng = np.random.default_rng(5)
+    lights = []
+    while len(lights) < 12:
+        L = np.array([rng.uniform(0.99, 1.0), *rng.uniform(-2e-3, 2e-3, 2)]).astype(f)
+        if abs(light_of(L, False) / light_of(L, True) - 1) > 0.02:
+            lights.append(L)
+    for L in lights:
+        arr = (abi.Light * 1)()
+        arr[0].color[:] = [1.0, 1.0, 1.0, 1.0]
+        arr[0].direction[:] = [-float(L[0]), -float(L[1]), -float(L[2]), 0.0]
+        arr[0].intensity, arr[0].type = 1.0, abi.LIGHT_DIRECTIONAL
+        sc.set_lights(arr)
+        for k in range(sc.n_draws):  # every tile, also those facing away from the light
+            sc.draws_host[k].lightMask = 1
+        sc.draws = to_device(sc.draws_host)
+        sc.light_cache.zero_()
+        sc.light(ds, passes=abi.SURFACE_DIRECT, camera=(4.0, 0.0, 0.0), shadow_bias=0.03)
+        torch.cuda.synchronize()
+        got = sc.light_cache.cpu().numpy()
+        drawn = got[..., 3] == 1.0
+        assert drawn.sum() == sc.n_draws * 64
+        np.testing.assert_allclose(got[drawn][:, :3], light_of(L, True), rtol=1e-4)
+
+
 def test_surface_emissive_pass_is_exact():
     from luxgi_amd.ddgi import DeviceScene
     from luxgi_amd.surface import SurfaceCache

@@ -259,6 +259,72 @@ def test_cell_records_hold_the_clamped_corners(shape, storage):
     assert np.all(rec[~written] == 0)  # padding records of partial bricks
 
 
+@pytest.mark.parametrize("layout,storage", [(abi.LAYOUT_LINEAR, abi.STORAGE_FP32), (abi.LAYOUT_LINEAR, abi.STORAGE_FP16),
+                                            (abi.LAYOUT_BRICK4, abi.STORAGE_FP32), (abi.LAYOUT_CELL8, abi.STORAGE_FP32),
+                                            (abi.LAYOUT_CELL8, abi.STORAGE_FP16)])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_outer_half_voxel_reads_the_edge_voxel_alone(axis, layout, storage):
+    """Within half a voxel of a face a lookup is the edge voxel's value (clamp to edge), whatever the voxel
+    behind it holds: rays along the faces across `axis`, a quarter voxel inside the volume, hit the same slab at
+    the same distance, bit for bit, whether the voxels between the two faces are finite or infinite, and
+    so in the oracle. So does the ray along an edge value that is infinite itself: it is far from any surface."""
+    from luxgi_amd.ddgi import DDGIVolume, DeviceScene
+    _, _, _, g, atlas = _scenes.small_scene()
+    along, across = (axis + 1) % 3, (axis + 2) % 3  # the ray's axis, and the third one
+
+    def field(n, behind, third):
+        pos = (np.arange(n) + 0.5) / n * 2.0 - 1.0
+        v = np.empty((n, n, n), np.float32)  # [z][y][x]
+        shape = [1, 1, 1]
+        shape[2 - along] = n
+        v[...] = ((0.5 - pos) / 2.0).astype(np.float32).reshape(shape)  # the slab along > 0.5, by the extent 2
+        cut = [slice(None)] * 3
+        if behind is not None:
+            cut[2 - axis] = slice(1, n - 1)
+            v[tuple(cut)] = behind
+        if third is not None:  # the upper face across the third axis
+            cut = [slice(None)] * 3
+            cut[2 - across] = n - 1
+            v[tuple(cut)] = third
+        return v
+
+    def trace(behind, third=None):
+        at = [0.0, 0.0, 0.0]
+        step = [1.0, 1.0, 1.0]
+        counts = [1, 1, 1]
+        at[along] = -0.75
+        at[axis], step[axis], counts[axis] = -1.0 + 0.25 / 32, 2.0 - 0.5 / 32, 2  # a quarter voxel inside both faces
+        at[across], step[across], counts[across] = 0.015625, 1.0 - 0.015625 - 0.25 / 32, 2  # mid, and its upper face
+        u = abi.make_uniform(tuple(counts), tuple(at), tuple(step), 1)
+        p = _scenes.trace_params()
+        rot = np.eye(4)
+        rot[:3, 0], rot[:3, along] = rot[:3, along].copy(), rot[:3, 0].copy()  # +x, the one ray, becomes `along`
+        p.randomOrientation = abi.mat4_colmajor(rot)
+        sdf, mip = field(64, behind, third), field(16, behind, third)
+        ds = DeviceScene(g, sdf, mip, atlas, layout=layout, sdf_storage=storage)
+        vol = DDGIVolume(u, flags_buffer=True)
+        vol.trace_rays(ds, p)
+        torch.cuda.synchronize()
+        if storage == abi.STORAGE_FP16:
+            sdf, mip = (v.astype(np.float16).astype(np.float32) for v in (sdf, mip))
+        ref = _scenes.oracle_trace(u, g, sdf, mip, atlas, p)
+        d, fl = vol.dir_dist.cpu().numpy()[:4, 0], vol.ray_flags.cpu().numpy()[:4, 0]
+        want = np.zeros(3)
+        want[along] = 1.0
+        np.testing.assert_allclose(d[:, :3], np.tile(want, (4, 1)), atol=1e-6)
+        assert np.array_equal(fl, ref[2][:4, 0])
+        np.testing.assert_allclose(d[:, 3], ref[1][:4, 0, 3], rtol=1e-4)
+        return d, fl
+
+    finite = trace(None)
+    assert np.all(finite[1] == 1)  # all four rays hit the slab
+    for a, b in zip(finite, trace(np.inf)):
+        assert np.array_equal(a, b)
+    d, fl = trace(None, third=np.inf)  # the probes at the third axis's face see nothing, the others as before
+    upper = (np.arange(4).reshape([2, 2]) // (2 if across > axis else 1)) % 2 == 1
+    assert np.array_equal(fl == 0, upper.reshape(-1)) and np.array_equal(d[fl == 1], finite[0][fl == 1])
+
+
 def test_trace_fp16_rays():
     prims, sdf, mip, g, atlas = _scenes.small_scene()
     u = _scenes.small_uniform(rays=64, counts=(4, 4, 4))

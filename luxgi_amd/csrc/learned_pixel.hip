@@ -234,8 +234,9 @@ __device__ __forceinline__ float lp_weight(const LpPassArgs& A, float cd, float 
 }
 
 // record[p] = (dL/d out_p / sw_p (rgb), s_p / phi_p) for filtered centres; mode[p]; dL/ds_p. One walk over
-// the taps: with r = dL/d out / sw and dw/ds = -|l_p - l_q| / phi_p w,
-// dL/ds = sum r . (x_q - out) dw/ds = -(1 / phi_p) (r . sum w |dl| x_q - (r . out) sum w |dl|).
+// the taps: with r = dL/d out / sw, dw/ds = -|l_p - l_q| / phi_p w and colours relative to the centre's (d_q =
+// x_q - x_p, m = sum w d_q / sw), dL/ds = sum r . (x_q - out) dw/ds = -(1 / phi_p) r . (sum w |dl| d_q - m sum w |dl|).
+// Sums of the colours themselves would cancel: a channel of 1000 that varies by 0.05 came out 1e-2 wrong.
 template <bool TILED>
 __global__ __launch_bounds__(256) void lp_pass_centre_kernel(LpPassArgs A, const float4* __restrict__ normals,
                                                              const float4* __restrict__ pbr,
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(256) void lp_pass_centre_kernel(LpPassArgs A, const
         cn = load_normal(normals, e);
     }
     float sw = 1.0f, sd = 0.0f;
-    f3 o = mk(c.x, c.y, c.z), od = mk(0.f, 0.f, 0.f);
+    f3 m1 = mk(0.f, 0.f, 0.f), md = m1;  // sums of w d_q and of w |dl| d_q
     for (int yy = -A.radius; yy <= A.radius; ++yy)
         for (int xx = -A.radius; xx <= A.radius; ++xx) {
             const int px = x + xx * A.stepSize, py = y + yy * A.stepSize;
@@ -315,15 +316,16 @@ __global__ __launch_bounds__(256) void lp_pass_centre_kernel(LpPassArgs A, const
             const float wd = w * fabsf(cl - sl);
             sw += w;
             sd += wd;
-            o = o + mk(sc.x, sc.y, sc.z) * w;
-            od = od + mk(sc.x, sc.y, sc.z) * wd;
+            const f3 dq = mk(sc.x - c.x, sc.y - c.y, sc.z - c.z);
+            m1 = m1 + dq * w;
+            md = md + dq * wd;
         }
     const float isw = 1.0f / sw;
-    o = o * isw;
+    const f3 k = md - m1 * (isw * sd);
     const float4 g = gOut[e];
     const f3 rr = mk(g.x * isw, g.y * isw, g.z * isw);
     record[e] = make_float4(rr.x, rr.y, rr.z, invPhiL);
-    gScale[e] = -invPhiC * (rr.x * (od.x - o.x * sd) + rr.y * (od.y - o.y * sd) + rr.z * (od.z - o.z * sd));
+    gScale[e] = -invPhiC * (rr.x * k.x + rr.y * k.y + rr.z * k.z);
 }
 
 // dL/d in_q (rgb): its own term plus r_p w_pq for every filtered neighbour p whose tap q is. Tiled, the

@@ -176,6 +176,40 @@ def test_pass_backward_at_block_edges_and_both_footprints(W, H, radius, step, ph
     assert np.allclose(b, ws_, rtol=1e-3, atol=1e-4 * np.abs(ws_).max()), np.abs(b - ws_).max()
 
 
+@pytest.mark.parametrize("radius,step", [(1, 1), (1, 16), (2, 4)])
+def test_scale_gradient_keeps_small_differences_of_a_bright_channel(radius, step):
+    """dL/ds sums r . (x_q - out) over the taps. A blue channel of 1000 that varies by 0.05, the only one with a
+    gradient, beside red and green that set the weights: the terms are differences 2e4 times smaller than their
+    operands. Relative to the centre texel the differences are exact in FP32 (neighbours within a factor of
+    two) and what remains are the roundings of the weights (the exponent |dl| s / phi <= 20 in FP32, its luminances
+    near 75: 1e-5) and of two sums that cancel to about a third: 1e-4 of the 2-norm. Sums of the colours
+    themselves lose 1000 x 6e-8 x sum w |dl| each, 2e-3 of it and more."""
+    from luxgi_amd._lib import lib
+    from luxgi_amd.ddgi import ptr, stream_handle
+    W, H = 61, 37
+    g, img, _, _ = _inputs(W, H, 31)
+    gd, gb = _gb(g)
+    rng = np.random.default_rng(32)
+    img[..., :2] = rng.uniform(0.0, 5.0, (H, W, 2))
+    img[..., 2] = 1000.0 + rng.uniform(-0.05, 0.05, (H, W))
+    img = img.astype(np.float32)
+    tiles = np.ones(lib().luxgi_svgf_tile_count(W, H), np.uint8)
+    sc = np.exp(rng.uniform(-0.5, 0.5, (H, W))).astype(np.float32)
+    go = np.zeros((H, W, 4), np.float32)
+    go[..., 2] = rng.normal(size=(H, W))
+    ap = abi.ReflectionAtrousParams(radius, step, 10.0, 32.0, 1.0, 1)
+    gin = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    gsc = torch.zeros((H, W), dtype=torch.float32, device="cuda")
+    ws = torch.empty(lib().luxgi_learned_pixel_pass_backward_workspace_size(W, H), dtype=torch.uint8, device="cuda")
+    assert lib().luxgi_learned_pixel_pass_backward(C.byref(ap), W, H, C.byref(gb), ptr(_dev(tiles)), ptr(_dev(img)),
+                                                   ptr(_dev(sc)), ptr(_dev(go)), ptr(gin), ptr(gsc), ptr(ws),
+                                                   ws.numel(), stream_handle()) == 0
+    torch.cuda.synchronize()
+    _, want = oracle.learned_pixel_atrous_backward(ap, W, H, g["normals"], g["pbr"], tiles, img, sc, go)
+    assert (want != 0).sum() > 200
+    assert np.linalg.norm(gsc.cpu().numpy() - want) <= 1e-4 * np.linalg.norm(want)
+
+
 def test_mlp_backward_matches_the_oracle_and_is_deterministic():
     from luxgi_amd._lib import lib
     from luxgi_amd.ddgi import ptr, stream_handle

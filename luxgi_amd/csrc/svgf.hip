@@ -36,30 +36,55 @@ struct GBuf {
 };
 
 
+// Unprojection of one image coordinate (worldPositionFromDepth, Common/Math.glsl:35-42): the clip position of
+// depth d is a + d b, with a of the coordinate and b, the matrix's third column, of the frame. The fused products
+// are named, so that the pixel and a tap at its coordinate and depth come out alike bit for bit.
+struct Unproject {
+    f3 a;
+    float aw;
+    const float* vpi;
+};
+__device__ __forceinline__ Unproject unproject_at(float u, float v, const float* vpi) {
+    const float x = u * 2.0f - 1.0f, y = v * 2.0f - 1.0f;
+    auto row = [&](int k) { return __builtin_fmaf(vpi[k], x, __builtin_fmaf(vpi[4 + k], y, vpi[12 + k])); };
+    return {mk(row(0), row(1), row(2)), row(3), vpi};
+}
+__device__ __forceinline__ float4 unproject(const Unproject& t, float depth) {
+    const float* b = t.vpi + 8;
+    return make_float4(__builtin_fmaf(depth, b[0], t.a.x), __builtin_fmaf(depth, b[1], t.a.y),
+                       __builtin_fmaf(depth, b[2], t.a.z), __builtin_fmaf(depth, b[3], t.aw));
+}
+__device__ __forceinline__ f3 unproject_point(float u, float v, float depth, const float* vpi) {
+    const float4 c = unproject(unproject_at(u, v, vpi), depth);
+    return mk(c.x / c.w, c.y / c.w, c.z / c.w);
+}
+
+// The same of the virtual point's ray: its history pixel is a truncated coordinate, which the last bit moves by
+// a pixel where a still or evenly panning view keeps it near a whole number, so the roundings are spelled out.
+__device__ __forceinline__ f3 virtual_ray_point(float u, float v, float depth, const float* m) {
+#pragma clang fp contract(off)
+    const float x = u * 2.0f - 1.0f, y = v * 2.0f - 1.0f;
+    float c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = (__builtin_fmaf(m[k], x, m[4 + k] * y) + m[8 + k] * depth) + m[12 + k];
+    return mk(c[0] / c[3], c[1] / c[3], c[2] / c[3]);
+}
+
 // isValid (Reprojection.glsl:42-53) of the taps of one pixel, with the pixel's part worked out once. The
-// reference unprojects every tap's depth pd at the pixel's history coordinate: a point
-// (a + pd b).xyz / (a + pd b).w with a and b fixed for the pixel, of which the plane test needs the
-// component along the pixel's normal only, so a tap costs two multiply-adds and a reciprocal; its
-// normal enters the angle test unnormalised, against |n|^2.
+// reference unprojects every tap's depth at the pixel's history coordinate and takes its distance to the
+// pixel's plane: (wpos - c.xyz / c.w) . n, here as (wpos c.w - c.xyz) . n against the limit times c.w, each
+// difference rounded once. (Projected on the normal first, wpos . n - c.xyz . n / c.w, the test is shorter by
+// half, but far from the origin it is the difference of two large numbers: at 1e5 units a still frame lost the
+// history of 30% of its pixels.) A tap's normal enters the angle test unnormalised, against |n|^2.
 struct TapTest {
-    f3 n;
-    float meshId, along;        // mesh id, wpos . n
-    float an, aw, bn, bw;       // a and b along n, and their w
+    f3 n, wpos;
+    float meshId;
+    Unproject at;               // the history coordinate
     bool inImage;               // the history pixel lies in the image
 };
 __device__ __forceinline__ TapTest tap_test(int hx, int hy, int W, int H, f3 wpos, f3 n, float meshId, float htx,
                                             float hty, const float* vpi) {
-    const float4 a = mat4_mul4(vpi, make_float4(htx * 2.0f - 1.0f, hty * 2.0f - 1.0f, 0.0f, 1.0f));
-    TapTest t;
-    t.n = n;
-    t.meshId = meshId;
-    t.along = dot3(wpos, n);
-    t.an = dot3(mk(a.x, a.y, a.z), n);
-    t.aw = a.w;
-    t.bn = dot3(mk(vpi[8], vpi[9], vpi[10]), n);
-    t.bw = vpi[11];
-    t.inImage = !(hx < 0 || hy < 0 || hx > W - 1 || hy > H - 1);
-    return t;
+    return {n, wpos, meshId, unproject_at(htx, hty, vpi), !(hx < 0 || hy < 0 || hx > W - 1 || hy > H - 1)};
 }
 struct TapTexel {
     float2 normal;
@@ -77,8 +102,10 @@ __device__ __forceinline__ TapTexel load_tap(const GBuf& prev, int x, int y, int
 }
 __device__ __forceinline__ bool is_valid(const TapTest& t, const TapTexel& p) {
     if (!t.inImage || t.meshId != p.meshId) return false;
-    const float prevAlong = (t.an + p.depth * t.bn) * __builtin_amdgcn_rcpf(t.aw + p.depth * t.bw);
-    if (fabsf(t.along - prevAlong) > kPlaneDistance) return false;
+    const float4 c = unproject(t.at, p.depth);
+    const f3 r = mk(__builtin_fmaf(t.wpos.x, c.w, -c.x), __builtin_fmaf(t.wpos.y, c.w, -c.y),
+                    __builtin_fmaf(t.wpos.z, c.w, -c.z));
+    if (fabsf(dot3(r, t.n)) > kPlaneDistance * fabsf(c.w)) return false;
     const f3 pn = oct_direction(p.normal.x, p.normal.y);
     const float d = dot3(t.n, pn);
     return !(d * d <= kNormalDistance * dot3(pn, pn));
@@ -138,13 +165,13 @@ __device__ bool reproject_rgb(const RA& A, int cx, int cy, float depth, float ra
     const float tcx = (float(cx) + 0.5f) / sx, tcy = (float(cy) + 0.5f) / sy;
     const float4 normal = fetch4(cur.normals, cx, cy, W, H);
     const float mx = normal.z, my = normal.w;
-    const f3 wpos = world_from_depth(tcx, tcy, depth, A.pc.viewProjInv);
+    const f3 wpos = unproject_point(tcx, tcy, depth, A.pc.viewProjInv);
     const float meshId = fetch4(cur.color, cx, cy, W, H).w;
     const float curvature = fetch4(cur.pbr, cx, cy, W, H).z;
     const float htx = tcx + mx, hty = tcy + my;
     float rx = float(cx) + mx * sx, ry = float(cy) + my * sy;
     if (rayLength > 0.0f && curvature == 0.0f) {  // virtualPointReprojection (Reprojection.glsl:56-75)
-        const f3 ro = world_from_depth(float(cx) / sx, float(cy) / sy, depth, A.pc.viewProjInv);
+        const f3 ro = virtual_ray_point(float(cx) / sx, float(cy) / sy, depth, A.pc.viewProjInv);
         const f3 cp = mk(A.pc.cameraPos[0], A.pc.cameraPos[1], A.pc.cameraPos[2]);
         f3 cr = ro - cp;
         const float cl = len3(cr);
@@ -627,7 +654,7 @@ __device__ bool reproject_scalar(const ShadowArgs& A, int cx, int cy, float dept
     const float tcx = pcx / sx, tcy = pcy / sy;
     const float4 normal = fetch4(cur.normals, cx, cy, W, H);
     const float mx = normal.z, my = normal.w;
-    const f3 wpos = world_from_depth(tcx, tcy, depth, A.pc.viewProjInv);
+    const f3 wpos = unproject_point(tcx, tcy, depth, A.pc.viewProjInv);
     const float meshId = fetch4(cur.color, cx, cy, W, H).w;
     const int hx = int(pcx + mx * sx), hy = int(pcy + my * sy);
     const float fx = floorf(float(cx)) + mx * sx, fy = floorf(float(cy)) + my * sy;

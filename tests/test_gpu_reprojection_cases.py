@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 import oracle
+from luxgi_amd import abi
 from tests.test_oracle_reprojection import (_checker, _gbuf, _hmom, _mask_from_bits, _refl, _shadow)
 
 pytestmark = pytest.mark.gpu
@@ -166,3 +167,54 @@ def test_shadow_reproject_closed_form_cases(case):
     assert np.array_equal(tiles.cpu().numpy(), rt_)
     np.testing.assert_allclose(oc.cpu().numpy(), rc_, rtol=0, atol=2e-5, err_msg=name)
     np.testing.assert_allclose(om.cpu().numpy(), rm_, rtol=0, atol=2e-5, err_msg=name)
+
+
+@pytest.mark.parametrize("kind", ["reflection", "shadow"])
+def test_a_still_frame_keeps_its_history_far_from_the_origin(kind):
+    """A still camera at (1e5, 3e4, 7e4): every pixel's own tap is the point itself, so its plane distance is 0 and
+    the history stays, though FP32 positions there are 8 mm apart and a tap unprojected by other roundings
+    lands metres away (1e5 x 6e-8 x depth / near plane, 20-500 units over 0.1). Every pixel has a mesh id of its
+    own, so no neighbour stands in for it. The distance that may remain is half a position's ulp in each
+    component, 4 mm x sqrt(3) against the reference's 5 units; the oracle keeps every pixel too."""
+    from luxgi_amd import _lib, scene
+    from luxgi_amd.ddgi import ptr, stream_handle
+    from luxgi_amd.svgf import gbuffer_struct
+    from tests._svgf_inputs import dir_to_oct
+    W, H = 61, 45
+    rng = np.random.default_rng(4)
+    eye = np.array([1e5, 3e4, 7e4])
+    P = scene.perspective_zo(np.pi / 3, W / H, 0.1, 1000.0)
+    vpi = np.linalg.inv(P @ scene.look_at(eye, eye + [0.3, -0.2, -1.0]))
+    z = np.exp(rng.uniform(np.log(20.0), np.log(500.0), (H, W)))
+    n = rng.normal(size=(H, W, 3))
+    g = {k: np.zeros((H, W, 4), np.float32) for k in ("color", "normals", "pbr")}
+    g["color"][..., 3] = 1.0 + np.arange(W * H).reshape(H, W)
+    g["normals"][..., :2] = dir_to_oct(n / np.linalg.norm(n, axis=-1, keepdims=True))
+    g["pbr"][..., 1], g["pbr"][..., 2], g["pbr"][..., 3] = 0.2, 1.0, z
+    g["depth"] = ((-P[2, 2] * z + P[2, 3]) / z).astype(np.float32)
+    hmom = _hmom(W, H, length=7.0)
+    dg, dmom = _dev(g), torch.from_numpy(hmom).cuda()
+    om = torch.zeros((H, W, 4), device="cuda")
+    tiles = torch.zeros(_lib.lib().luxgi_svgf_tile_count(W, H), dtype=torch.uint8, device="cuda")
+    gb = gbuffer_struct(dg)
+    if kind == "reflection":
+        p = _refl()
+        p.viewProjInv = abi.mat4_colmajor(vpi)
+        sig, hist = np.full((H, W, 4), 0.5, np.float32), np.full((H, W, 4), 0.5, np.float32)
+        sig[..., 3] = 0.0  # no ray length: the pixel's own position, not the virtual point
+        oc = torch.zeros((H, W, 4), device="cuda")
+        call, ref = _lib.lib().luxgi_svgf_reflection_reproject, oracle.reflection_reproject
+    else:
+        p = _shadow()
+        p.viewProjInv = abi.mat4_colmajor(vpi)
+        sig, hist = _mask_from_bits(np.ones((H, W), np.uint8)), np.full((H, W, 2), 0.5, np.float32)
+        oc = torch.zeros((H, W, 2), device="cuda")
+        call, ref = _lib.lib().luxgi_svgf_shadow_reproject, oracle.shadow_reproject
+    dsig = torch.from_numpy(sig if kind == "reflection" else sig.view(np.int32)).cuda()
+    dhist = torch.from_numpy(hist).cuda()
+    assert call(C.byref(p), W, H, 0, C.byref(gb), C.byref(gb), ptr(dsig), ptr(dhist), ptr(dmom), ptr(oc), ptr(om),
+                ptr(tiles), stream_handle()) == 0
+    torch.cuda.synchronize()
+    assert np.all(ref(p, W, H, g, g, sig, hist, hmom)[1][..., 2] == 8.0)
+    lost = om.cpu().numpy()[..., 2] != 8.0
+    assert not lost.any(), lost.mean()

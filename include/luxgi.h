@@ -123,8 +123,7 @@ typedef struct LuxgiTraceParams {
     /* --- extensions (defaults reproduce the reference) --- */
     int32_t  maxSteps;      /* per-cascade step cap; reference = 250 (SDFCommon.glsl:143) */
     float    hitEpsilon;    /* 0 = reference thickness test (SDFCommon.glsl:166-167); >0 = fixed eps */
-    int32_t  shadeOrder;    /* 0 or 1. Both shade in ray order, a wave's hits grouped as it goes (0 once sorted
-                               the hits by surface-atlas chunk); the outputs are identical */
+    int32_t  shadeOrder;    /* 0 or 1, other values are refused; selects nothing: both run the same kernels */
     int32_t  pad1;
     float    skyColor[4];   /* sky radiance when no cubemap is bound (reference binds a unit cube) */
     const float* deviceOrientation; /* optional device array of 16 floats (column-major): read in place of

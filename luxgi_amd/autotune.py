@@ -106,8 +106,9 @@ def tune_svgf_batch(batch, tuner=None, check=True):
 
 
 def tune_trace_shade_order(volume, scene, params, tuner=None):
-    """Times the trace's two shadeOrder values for a DDGIVolume and scene (both shade in ray order and give
-    identical ray data), sets params.shadeOrder to the faster and returns it."""
+    """Times the trace for the two values that shadeOrder accepts, sets params.shadeOrder to the one that came
+    out and returns it. Both run the same kernels, so there is nothing to gain: kept for programs that
+    call it."""
     tuner = tuner or Autotuner()
     u = volume.u
     sig = f"{u.probeCounts[0]}x{u.probeCounts[1]}x{u.probeCounts[2]}x{u.raysPerProbe}|{scene.n_objects}"

@@ -67,8 +67,8 @@ struct TraceArgs {
 
 // ---------------------------------------------------------------------------
 // March (tracyGlobalSDF, SDFCommon.glsl:98-194): one lane per ray, the 64 lanes
-// of a wave on 64 rays of one probe, in trace_block's order. A front hit's record (hitTime, texture UV of the hit step; cascade)
-// goes to the workspace for shade_kernel.
+// of a wave on 64 rays of one probe, in trace_block's order. A front hit's record (hitTime, texture
+// UV of the hit step; cascade) goes to the workspace for shade_kernel.
 // ---------------------------------------------------------------------------
 
 __device__ __forceinline__ void ray_setup(const TraceArgs& A, const LuxgiTraceVolume& v, int probe, int ray,
@@ -417,16 +417,17 @@ __global__ __launch_bounds__(256) void march_kernel(TraceArgs A, float4* __restr
 // One lane per hit, with the hits counting-sorted by chunk so that a wave's lists agree, took
 // 479 us for the 2.4 M hits of a 32x16x32x256 volume and 300 us more for the sort: its keys, a
 // histogram with an atomic per chunk of each wave, a scan, a scatter, and records and outputs at
-// scattered addresses; the whole trace 1,652 us against 1,513 now (shade 487), 102 against 68 for a
-// 13x7x11x100 volume in FP16 and 120 against 90 for an 8x8x8x64 one. Bound at the large size: L2
-// misses (19.6 M lines in 487 us, 5.1 TB/s), a third of them the normals'.
+// scattered addresses. The whole trace took 1,652 us so and 1,513 in this form (shade 487), before
+// trace_block's runs made it 1,350; a 13x7x11x100 volume in FP16 102 and 68, an 8x8x8x64 one 120 and 90, before
+// kFewRays made the last 67. Bound at the large size: L2 misses (19.6 M lines in 487 us, 5.1 TB/s), a third
+// of them the normals'.
 template <class SS, class SC, class SR, bool COUNT, int MODE>
 __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __restrict__ objInvBase,
                                                     const float4* __restrict__ recA, const uint8_t* __restrict__ recC,
                                                     unsigned long long* __restrict__ counters) {
     __shared__ AtlasQueryLds lds[4];
     const long long gid = wave_ray(A);
-    Counts c = {0, 0, 0, 0, 0, 0, 0};
+    Counts c{};
     const LuxgiTraceVolume* v;
     int probe, ray;
     size_t rid;
@@ -521,10 +522,20 @@ extern "C" size_t luxgi_ddgi_trace_workspace_size(const LuxgiDDGIUniform* u, int
     return trace_workspace_layout(P * R, objectCapacity, nullptr, nullptr);
 }
 
-// Up to this many rays a wave takes 16 of them. A small trace is the chain of its longest rays and of its
-// waves' hits, eight at a time, with most of the chip idle: shorter waves spread the hits over four
-// times as many. 4,096 rays 86 -> 66 us, 32,768 87 -> 67, 65,536 92 -> 82; 100,100 rays already
-// lose by it (64 -> 75) and 196,608 more (74 -> 94).
+// Up to this many rays (counted as lanes: a single volume's rays per probe padded to a multiple of 64) a wave
+// takes 16 of them. A small trace is the chain of its longest rays and of its waves' hits, eight at a time,
+// with most of the chip idle: shorter waves spread the hits over four times as many. Full waves -> short ones, us,
+// for 32,768 lanes (8x8x8x64) and 65,536 (16x8x8x64), then 76,800, 98,304 (12x8x16x64) and 131,072
+// (16x8x16x64), 300 objects:
+//   linear FP32 256^3  83 -> 75, 86 -> 80, 102 -> 90, 109 -> 99, 119 -> 126   64^3  50 -> 44, 50 -> 50, 51 -> 55
+//   cells FP32 256^3   63 -> 57, 63 -> 61, 64 -> 62, 68 -> 68, 74 -> 87       64^3  47 -> 38, 51 -> 47, 53 -> 49
+//   bricks FP32 128^3  60 -> 55, 63 -> 63, 69 -> 66, 74 -> 75, 74 -> 94
+//   linear FP16 128^3  57 -> 49, 59 -> 59, 77 -> 68, 79 -> 72, 82 -> 88
+//   cells FP16 128^3   54 -> 49, 55 -> 55, 58 -> 60, 60 -> 64, 63 -> 79
+//   bricks FP16 128^3  56 -> 50, 61 -> 59, 65 -> 64, 67 -> 69, 69 -> 86
+// Batches of three volumes, update included: 33,028 rays 98 -> 92, 57,344 93 -> 91, 81,920 97 -> 95,
+// 100,352 102 -> 118; over two scenes 98 -> 91, 89 -> 88, 99 -> 94, 102 -> 110. Up to 65,536 none loses more
+// than 1%, past it the forms part.
 constexpr long long kFewRays = 65536;
 
 // The kernels of one trace: object inverses, march, shade. MODE 0: one volume, 1: a batch over A.scene,
@@ -620,7 +631,7 @@ static int trace_scene_descriptor(const LuxgiGlobalSDFData* g, const LuxgiSDFVol
 // The scene arguments shared by the single and batched traces: checks them and fills A's scene
 // and the call's settings.
 static int trace_scene_args(const LuxgiGlobalSDFData* g, const LuxgiSDFVolume* vol, const LuxgiSurfaceAtlas* at,
-                            const LuxgiSkybox* sky, const LuxgiTraceParams* p, bool count, TraceArgs& A) {
+                            const LuxgiSkybox* sky, const LuxgiTraceParams* p, TraceArgs& A) {
     if (!p) return LUXGI_ERR_INVALID_ARGUMENT;
     const int rc = trace_scene_descriptor(g, vol, at, sky, p->skyColor, A.scene);
     if (rc != LUXGI_OK) return rc;
@@ -684,7 +695,7 @@ static int trace_entry(const LuxgiDDGIUniform* u, const LuxgiGlobalSDFData* g, c
     int rc = trace_volume_ok(u, rays);
     if (rc != LUXGI_OK) return rc;
     TraceArgs A;
-    rc = trace_scene_args(g, vol, at, sky, p, COUNT, A);
+    rc = trace_scene_args(g, vol, at, sky, p, A);
     if (rc != LUXGI_OK) return rc;
     A.P = u->probeCounts[0] * u->probeCounts[1] * u->probeCounts[2];
     A.R = u->raysPerProbe;
@@ -734,7 +745,7 @@ extern "C" int luxgi_ddgi_trace_sdf_batched(const LuxgiTraceVolume* volumes, int
     if (!volumes || count <= 0 || count > LUXGI_MAX_TRACE_BATCH || totalRays <= 0 || totalRays >= (1ll << 31))
         return LUXGI_ERR_INVALID_ARGUMENT;
     TraceArgs A;
-    const int rc = trace_scene_args(g, vol, at, sky, p, false, A);
+    const int rc = trace_scene_args(g, vol, at, sky, p, A);
     if (rc != LUXGI_OK) return rc;
     A.P = A.R = A.rayWidth = 0;
     A.vols = volumes;

@@ -11,9 +11,6 @@ __device__ __forceinline__ bool inside(int x, int y, int W, int H) { return x >=
 __device__ __forceinline__ float4 fetch4(const float4* p, int x, int y, int W, int H) {
     return inside(x, y, W, H) ? p[(size_t)y * W + x] : make_float4(0.f, 0.f, 0.f, 0.f);
 }
-__device__ __forceinline__ float fetch1(const float* p, int x, int y, int W, int H) {
-    return inside(x, y, W, H) ? p[(size_t)y * W + x] : 0.0f;
-}
 template <class S>
 __device__ __forceinline__ float4 fetchS4(const S* p, int x, int y, int W, int H) {
     return inside(x, y, W, H) ? Texel<S>::ld4(p, (size_t)y * W + x) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -88,8 +85,10 @@ __device__ __forceinline__ f3 oct_direction(float ox, float oy) {
     }
     return v;
 }
-// a texel's normal: octahedral xy only, normalised with the reciprocal square root (v_rsq_f32, within
-// 1 ulp; the square root and three divisions it stands for were a tenth of an a-trous pass)
+// a texel's normal: octahedral xy only, normalised with the reciprocal square root (v_rsq_f32, within 1 ulp).
+// With the square root and three divisions that it stands for, 1920x1080: reflection frame 285 us against
+// 268, shadow frame 172 against 160. Frames against 64 bits: 3.2570e-4 and 2.0174e-4 either way (2-norm); a
+// typical shadow texel's rounding grows by 1% (1.239e-7 to 1.248e-7 without the worst tenth).
 __device__ __forceinline__ f3 load_normal(const float4* normals, size_t q) {
     const float2 o = reinterpret_cast<const float2*>(normals)[2 * q];
     const f3 v = oct_direction(o.x, o.y);

@@ -172,8 +172,8 @@ def test_ddgi_batch_graph_replay_matches_per_volume_updates(trace, streams, blen
 
 
 def test_autotuner_trace_shade_order(tmp_path):
-    """tune_trace_shade_order times both shading orders of the trace (identical outputs), sets the
-    fastest in the parameters and caches it."""
+    """tune_trace_shade_order times the two values that shadeOrder accepts (they run the same kernels, so either
+    may come out), sets the one it took in the parameters and caches it."""
     from luxgi_amd.autotune import Autotuner, tune_trace_shade_order
     from luxgi_amd.ddgi import DDGIVolume, DeviceScene
     from tests import _scenes
@@ -241,6 +241,36 @@ def test_several_scene_batch_matches_per_volume_traces_on_their_scenes(storage):
             assert torch.equal(other.current_depth, vol.current_depth)
     hits = [(v.dir_dist[..., 3] < 1000).float().mean().item() for v in singles]
     assert min(hits) > 0.03 and max(hits) < 0.95, hits  # the scenes are hit and missed
+
+
+@pytest.mark.parametrize("several", [False, True])
+def test_batched_traces_in_full_waves_equal_per_volume_traces(several):
+    """Batches above 65,536 rays trace 64 to a wave: five volumes of 69,273 rays together, over one scene and over
+    three (there each starts at a multiple of 64 rays), whose boundaries lie inside blocks and, over one
+    scene, inside waves, with a ragged tail. Each volume alone is below that line and traces 16 to a wave;
+    both give the same rays bit for bit."""
+    from luxgi_amd import scene
+    from luxgi_amd.batch import DDGIBatch
+    from luxgi_amd.ddgi import DDGIVolume, default_trace_params
+    from tests import _scenes
+    scenes = _scene_set()
+    scene_of = [0, 1, 2, 1, 0] if several else [0] * 5
+    unis = [_scenes.small_uniform(rays=100, counts=(7, 9, 5)), _scenes.small_uniform(rays=65, counts=(5, 5, 5)),
+            _scenes.small_uniform(rays=96, counts=(9, 4, 8)), _scenes.small_uniform(rays=37, counts=(3, 3, 3)),
+            _scenes.small_uniform(rays=1, counts=(7, 11, 13))]
+    assert sum(u.num_probes * u.raysPerProbe for u in unis) == 69273
+    batch = DDGIBatch(unis, scenes if several else scenes[0], scene_of=scene_of if several else None)
+    rots = [scene.random_rotation(40 + k) for k in range(5)]
+    batch.update(rots)
+    for k, u in enumerate(unis):
+        assert u.num_probes * ((u.raysPerProbe + 63) // 64 * 64) <= 65536
+        vol = DDGIVolume(u)
+        vol.trace_rays(scenes[scene_of[k]], default_trace_params(rots[k], frame=0))
+        torch.cuda.synchronize()
+        print(f"volume {k} scene {scene_of[k]}", flush=True)
+        assert torch.equal(batch.volumes[k].radiance, vol.radiance)
+        assert torch.equal(batch.volumes[k].dir_dist, vol.dir_dist)
+        assert (vol.dir_dist[..., 3] < 1000).any()
 
 
 def test_several_scene_batch_rejects_mixed_storage_and_bad_scene_index():

@@ -145,8 +145,9 @@ def test_sdf_reflection_matches_oracle(layout, atlas_layout):
 @pytest.mark.parametrize("W,H", [(1, 1), (1, 300), (300, 1), (31, 33), (32, 256), (257, 40), (289, 95)])
 def test_sdf_reflection_traces_every_pixel_once_at_the_edges_of_its_pixel_squares(W, H):
     """Mirror rays over images below, at and past the 8x8 blocks, the 32x32 squares and the rows of eight of
-    them: pixels that are not sky agree with the oracle (the bounds of the test above; at least two
-    pixels may graze past a surface), sky pixels and the texels after the image keep their value."""
+    them: every pixel that is not sky is written, sky pixels and the texels after the image keep their value.
+    The written values agree with the oracle within the bounds of the test above: 1% of the pixels, and two
+    where there are more than 100, may graze past a surface; a single pixel may not."""
     from luxgi_amd.ddgi import DeviceScene, to_device
     from luxgi_amd.producers import BlueNoiseTables, sdf_reflection
     from luxgi_amd.svgf import make_gbuffer
@@ -174,5 +175,6 @@ def test_sdf_reflection_traces_every_pixel_once_at_the_edges_of_its_pixel_square
                                  sky_size=8, out=np.full((H, W, 4), -5.0))
     sky_px = depth == 1.0
     assert np.all(got[sky_px] == -5.0) and bool((whole[W * H:] == -5.0).all())
+    assert not np.any(np.all(got == -5.0, axis=-1)[~sky_px])
     ok = np.all(np.abs(got - want) <= 2e-3 * (1 + np.abs(want)), axis=-1)[~sky_px]
-    assert (~ok).sum() <= max(2, 0.01 * ok.size), ((~ok).sum(), ok.size)
+    assert (~ok).sum() <= max(2 if ok.size > 100 else 0, 0.01 * ok.size), ((~ok).sum(), ok.size)

@@ -86,11 +86,13 @@ def test_trace_matches_oracle_config1(max_steps, hit_eps):
     assert (fl == 1).mean() > 0.3 and (fl == 0).mean() > 0.01  # the scene has hits and misses
 
 
+@pytest.mark.parametrize("counts", [(9, 8, 7), (12, 11, 8)])
 @pytest.mark.parametrize("rays", [1, 7, 63, 65])
-def test_trace_shade_groups_at_wave_and_list_edges(rays):
-    """Waves with 1, 7, 63 and 64 + 1 rays (hits in partly filled groups of eight lanes) over a scene whose
-    chunks hold 1 to 16 objects (lists of 8, 9 and 16, the groups' steps). Tolerances as in the other
-    trace tests."""
+def test_trace_shade_groups_at_wave_and_list_edges(rays, counts):
+    """1, 7, 63 and 64 + 1 rays a probe (hits in partly filled groups of eight lanes) over a scene whose
+    chunks hold 1 to 16 objects (lists of 8, 9 and 16, the groups' steps): 504 probes, at most 64,512
+    padded rays, in waves of 16, and 1,056 probes, 67,584 padded rays and more, in waves of 64. Tolerances as
+    in the other trace tests."""
     prims = scene.scene_random(n=60, seed=9, size_range=(0.4, 1.0))
     sdf = scene.bake_sdf_numpy(prims, 64)
     g = abi.make_sdf_data(resolution=64)
@@ -98,7 +100,7 @@ def test_trace_shade_groups_at_wave_and_list_edges(rays):
     atlas = scene.build_atlas(prims, resolution=512, tile=16, seed=3, threshold=1.05 * 2.0 / 64)
     lists = set(atlas.culled[atlas.chunks[atlas.chunks > 0]].tolist())
     assert {1, 7, 8, 9, 16} <= lists
-    u = _scenes.small_uniform(rays=rays, counts=(9, 8, 7))
+    u = _scenes.small_uniform(rays=rays, counts=counts)
     p = _scenes.trace_params(rot_seed=17)
     gpu = _gpu_trace(u, g, sdf, mip, atlas, p)
     ref = _scenes.oracle_trace(u, g, sdf, mip, atlas, p)
@@ -127,25 +129,26 @@ def test_trace_is_the_same_for_short_and_full_waves(rays):
     assert (outs[0][2] == 1).mean() > 0.3
 
 
-@pytest.mark.parametrize("nz", [17, 25])
-def test_trace_is_the_same_for_blocks_dealt_in_runs_and_in_eighths(nz):
+@pytest.mark.parametrize("nx,ny,nz,part", [(31, 33, 17, 16), (31, 33, 25, 16), (32, 32, 16, 15)])
+def test_trace_is_the_same_for_blocks_dealt_in_runs_and_in_eighths(nx, ny, nz, part):
     """From 4,096 blocks of 256 padded rays on the XCDs take runs of 256 blocks, below that, and after the last
-    whole turn of 2,048, eighths. A volume past that line (one and two turns with a ragged tail) gives the texels
-    of its first and its last 16 layers, each traced below it, bit for bit; the probe positions are exact
-    binary fractions, so the parts see the same origins."""
+    whole turn of 2,048, eighths. A volume on that side of the line (two and three turns with a ragged tail, 4,348
+    and 6,394 blocks, and exactly two turns) gives the texels of its first and its last `part` layers, each
+    traced below it, bit for bit; the probe positions are exact binary fractions, so the parts see the
+    same origins."""
     from luxgi_amd.ddgi import DDGIVolume, DeviceScene
     prims, sdf, mip, g, atlas = _scenes.small_scene()
     ds = DeviceScene(g, sdf, mip, atlas)
     p = _scenes.trace_params(rot_seed=29)
 
     def trace(z0, n):
-        u = abi.make_uniform((31, 33, n), (-0.5, -0.5, -0.5 + z0 / 32), (1 / 32, 1 / 32, 1 / 32), 37)
+        u = abi.make_uniform((nx, ny, n), (-0.5, -0.5, -0.5 + z0 / 32), (1 / 32, 1 / 32, 1 / 32), 37)
         vol = DDGIVolume(u, flags_buffer=True)
         vol.trace_rays(ds, p)
         torch.cuda.synchronize()
-        return [t.cpu().numpy()[: 31 * 33 * n] for t in (vol.radiance, vol.dir_dist, vol.ray_flags)]
+        return [t.cpu().numpy()[: nx * ny * n] for t in (vol.radiance, vol.dir_dist, vol.ray_flags)]
 
-    whole, first, last = trace(0, nz), trace(0, 16), trace(nz - 16, 16)
+    whole, first, last = trace(0, nz), trace(0, part), trace(nz - part, part)
     for w, a, b in zip(whole, first, last):
         assert np.array_equal(w[: len(a)], a) and np.array_equal(w[-len(b):], b)
     assert (whole[2] == 1).mean() > 0.05
@@ -165,8 +168,8 @@ def test_trace_unorm8_atlas_and_offsets():
 
 @pytest.mark.parametrize("order", [0, 1])
 def test_trace_sky_cubemap_matches_oracle(order):
-    """Misses sample the sky cube map (GISDFRays.comp:121-124); with the hit sort (order 0) the
-    march stores them, in ray order the shade pass does."""
+    """Misses sample the sky cube map (GISDFRays.comp:121-124) and are stored by the march, for both values
+    that shadeOrder accepts."""
     prims, sdf, mip, g, atlas = _scenes.small_scene()
     u = _scenes.small_uniform(rays=128, counts=(5, 4, 6))
     p = _scenes.trace_params(rot_seed=17)
@@ -444,9 +447,8 @@ def test_trace_fp16_scaled_bricks_and_fp32_refine_vs_oracle():
 
 @pytest.mark.parametrize("layout,guard", [(abi.LAYOUT_BRICK4, False), (abi.LAYOUT_LINEAR, True)])
 def test_trace_shade_order_is_bitwise_identical(layout, guard):
-    """Shading the front hits grouped by surface-atlas chunk (the default: the march writes the
-    misses and inside hits, a counting sort orders the rest) or every ray in ray order gives the
-    same outputs bit for bit; the counting trace (always in ray order) agrees too."""
+    """Both values that shadeOrder accepts give the same outputs bit for bit (they run the same kernels), and
+    so does the counting trace, whose kernels are others; a second call on the same workspace too."""
     from luxgi_amd.ddgi import DDGIVolume, DeviceScene
     prims, sdf, mip, g, atlas = _scenes.small_scene()
     u = _scenes.small_uniform(rays=96, counts=(7, 5, 6))
@@ -457,7 +459,7 @@ def test_trace_shade_order_is_bitwise_identical(layout, guard):
         ds = DeviceScene(g, sdf, mip, atlas, layout=layout, guard=guard)
         vol = DDGIVolume(u, flags_buffer=True)
         counters = torch.zeros(8, dtype=torch.int64, device="cuda") if count else None
-        for _ in range(2):  # the second call reuses the workspace: the bins must start from zero again
+        for _ in range(2):  # the second call reuses the workspace
             vol.trace_rays(ds, p, counters=counters)
         torch.cuda.synchronize()
         outs.append((vol.radiance.cpu().numpy(), vol.dir_dist.cpu().numpy(), vol.ray_flags.cpu().numpy()))

@@ -393,14 +393,14 @@ __global__ __launch_bounds__(256) void march_kernel(TraceArgs A, float4* __restr
     if (find_ray<MODE>(A, gid, v, probe, ray, rid) && lane_traces(A))
         march_ray<SS, SR, COUNT, FL>(A, MODE == 2 ? A.scenes[v->scene] : A.scene, *v, probe, ray, rid, recA, recC, cMip,
                                      cFine, cSteps, cHits);
-    if (COUNT) {
+    if (COUNT) {  // lanes without a count stay away from the LDS atomics, which serialise
         __shared__ unsigned long long sc[4];
         if (threadIdx.x < 4) sc[threadIdx.x] = 0;
         __syncthreads();
-        atomicAdd(&sc[0], cMip);
-        atomicAdd(&sc[1], cFine);
-        atomicAdd(&sc[2], cSteps);
-        atomicAdd(&sc[3], cHits);
+        if (cMip) atomicAdd(&sc[0], cMip);
+        if (cFine) atomicAdd(&sc[1], cFine);
+        if (cSteps) atomicAdd(&sc[2], cSteps);
+        if (cHits) atomicAdd(&sc[3], cHits);
         __syncthreads();
         if (threadIdx.x == 0) {
             atomicAdd(&counters[0], sc[0]);
@@ -472,10 +472,10 @@ __global__ __launch_bounds__(256) void shade_kernel(TraceArgs A, const float* __
         __shared__ unsigned long long sc[4];
         if (threadIdx.x < 4) sc[threadIdx.x] = 0;
         __syncthreads();
-        atomicAdd(&sc[0], c.normals);
-        atomicAdd(&sc[1], c.objects);
-        atomicAdd(&sc[2], c.tiles);
-        atomicAdd(&sc[3], valid ? 1ull : 0ull);
+        if (c.normals) atomicAdd(&sc[0], c.normals);
+        if (c.objects) atomicAdd(&sc[1], c.objects);
+        if (c.tiles) atomicAdd(&sc[2], c.tiles);
+        if (valid) atomicAdd(&sc[3], 1ull);
         __syncthreads();
         if (threadIdx.x < 4) atomicAdd(&counters[2 + threadIdx.x], sc[threadIdx.x]);
     }
@@ -544,7 +544,7 @@ template <class SS, class SC, class SR, bool COUNT, int MODE>
 static int launch_trace(TraceArgs A, int nScenes, int maxObjects, const TraceWorkspace& w,
                         unsigned long long* counters, hipStream_t st) {
     const long long lanes = MODE != 0 ? A.totalRays : (long long)A.P * ((A.R + 63) & ~63);
-    A.waveRays = lanes <= kFewRays ? 16 : 64;
+    A.waveRays = !COUNT && lanes <= kFewRays ? 16 : 64;
     if (MODE == 2) {
         if (maxObjects > 0) {
             hipLaunchKernelGGL(trace_prepare_scenes_kernel, dim3((maxObjects + 255) / 256, nScenes), dim3(256), 0, st,

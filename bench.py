@@ -807,7 +807,7 @@ def main():
                          "rays": n_rays, "steps": c[6], "hits": c[7]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "measured_copy_gbs": copy_gbs,
-                     "kernel": "luxgi_ddgi_trace_sdf launch sequence (march + hit sort + shade)",
+                     "kernel": "luxgi_ddgi_trace_sdf launch sequence (object inverses + march + shade)",
                      "algorithmic_bytes_per_launch": trace_bytes},
         "cpu_baseline": cpu,
     }

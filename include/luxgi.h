@@ -837,8 +837,8 @@ int luxgi_ddgi_trace_batch_prepare(LuxgiTraceVolume* volumes, int32_t count, int
 /* Workspace bytes of luxgi_ddgi_trace_sdf_batched for `totalRays` rays. */
 size_t luxgi_ddgi_trace_batch_workspace_size(int64_t totalRays, int32_t objectCapacity);
 
-/* luxgi_ddgi_trace_sdf for several volumes over one scene in one launch sequence: the march, the
- * hit sort and the shade each run once over the flat list of all volumes' rays, each ray finding
+/* luxgi_ddgi_trace_sdf for several volumes over one scene in one launch sequence: the march
+ * and the shade each run once over the flat list of all volumes' rays, each ray finding
  * its volume by binary search over rayStart. Every volume's outputs are identical to a
  * luxgi_ddgi_trace_sdf call on it. `volumes` is a device array of `count` prepared descriptors
  * (read when the kernels run); `params` gives the shared settings (maxSteps, hitEpsilon,
